@@ -15,9 +15,9 @@
 // SDF MLP consumes.  Forward: one thread per (point, level), level-minor, so
 // the L lanes of a point write its output row in one wave instruction (whole
 // cache lines; a level-major grid writes each row 16 bytes at a time from
-// workgroups launched far apart).  Backward: one thread per (point, feature) so the F
-// atomics of one corner are adjacent lanes of one instruction and coalesce
-// into a single L2 atomic request.
+// workgroups launched far apart).  Backward: a lane per (corner, feature), so the
+// F atomics of one entry, and the entries of an x pair, are adjacent lanes of one
+// instruction and coalesce into one L2 atomic request.
 #include <cstring>
 
 #include "common.h"
@@ -346,35 +346,110 @@ hashgrid_fwd_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n, floa
   RowStore<F, TO>::store(o, acc);
 }
 
+// F consecutive upstream gradients as floats; `vec`: the rows allow the vector load.
+template <int F, typename TD>
+__device__ inline void load_row(const TD* __restrict__ p, bool vec, float (&v)[F]) {
+  if (vec) {
+    EntryLoad<F, TD>::load(p, v);
+  } else {
+#pragma unroll
+    for (int f = 0; f < F; ++f) v[f] = scalar_io<TD>::load(p + f);
+  }
+}
+
+// Table gradient of one encoder evaluation per point.  The eight corners of a
+// point and their F features are the lanes of one instruction (64 / 8F points side by
+// side), so the two entries of an x pair go out as one request.  A lane does
+// not hold corner c of the current cell but the corner whose lattice coordinates
+// have the lane's parity: while consecutive points (samples of a ray) stay in a
+// cell, or move to one that shares corners, those lanes' entries do not change
+// and the sums stay in registers; a lane adds to memory only when its own entry
+// changes.  What a point needs is formed once, by one lane for 64 points at a
+// time, as per-axis, per-parity (weight, index term) pairs in LDS, which leaves
+// each lane three reads, two products and two adds (or xors) per point; with
+// every lane forming its own corner the coarse levels were VALU-bound.
+// One feature per lane and eight separate corner instructions (before): 6.24 ms at
+// 786,432 points, 2^22 x 16 x 8, bf16 gradients, and 1.84 ms at 262,147 points,
+// 2^19 x 16 x 4, float32.  Now 2.03 and 0.58 ms; a fine level costs the same
+// 0.16 ms per 786,432 points either way it is ordered (by ray, along a
+// space-filling curve, a level per XCD): the read-modify-write of its sectors
+// in L2 and behind it is the bound.
+constexpr int kBwdWaves = kBlock / 64;
+
 template <int F, typename TD>
 __global__ void __launch_bounds__(kBlock)
 hashgrid_bwd_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n, float vmin,
-                    float vrange, const TD* __restrict__ dy, int64_t ld,
-                    float* __restrict__ grad, int active) {
+                    float vrange, const TD* __restrict__ dy, int64_t ld, int vec,
+                    float* __restrict__ grad, int active, int run) {
+  constexpr int G = 64 / (8 * F);  // points side by side in a wave
+  __shared__ float2 s_axis[kBwdWaves][64][6];  // [axis * 2 + parity] = (weight, index term)
+  __shared__ float s_g[kBwdWaves][64][F];
   int64_t chunk;
   int l;
   chunk_level(active, chunk, l);
-  int64_t tid = chunk * kBlock + threadIdx.x;
-  int64_t i = tid / F;
-  int f = (int)(tid % F);
-  if (i >= n) return;
-  const int L = d.n_levels;
-  (void)L;
-  float g = scalar_io<TD>::load(dy + i * ld + l * F + f);
-  if (g == 0.0f) return;  // adding +0 leaves the accumulator unchanged
-  LevelParams p = level_params(d, l);
-  uint32_t cell[3];
-  float t[3];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int per_wave = G * run;  // <= 64
+  const int64_t i0 = (chunk * kBwdWaves + wave) * per_wave;
+  if (i0 >= n) return;  // whole waves: the LDS rows are a wave's own
+  const LevelParams p = level_params(d, l);
+  if (lane < per_wave) {
+    const int64_t i = i0 + lane;
+    float g[F];
 #pragma unroll
-  for (int k = 0; k < 3; ++k)
-    pos_fract(normalize_coord(x[i * 3 + k], vmin, vrange), p.scale, cell[k], t[k]);
+    for (int f = 0; f < F; ++f) g[f] = 0.0f;
+    if (i < n) {
+      load_row<F, TD>(dy + i * ld + l * F, vec != 0, g);
+      const uint32_t step[3] = {1u, p.hashed ? 2654435761u : p.res,
+                                p.hashed ? 805459861u : p.res * p.res};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        uint32_t cell;
+        float t;
+        pos_fract(normalize_coord(x[i * 3 + k], vmin, vrange), p.scale, cell, t);
+        const uint32_t term = cell * step[k];
+        const bool odd = (cell & 1u) != 0;
+        const float2 lo = make_float2(1.0f - t, __uint_as_float(term));
+        const float2 hi = make_float2(t, __uint_as_float(term + step[k]));
+        s_axis[wave][lane][2 * k] = odd ? hi : lo;
+        s_axis[wave][lane][2 * k + 1] = odd ? lo : hi;
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < F; ++f) s_g[wave][lane][f] = g[f];
+  }
+  __builtin_amdgcn_wave_barrier();
+  __threadfence_block();  // the wave's own LDS writes, before its reads
+  const int f = lane % F, c = (lane / F) & 7, first = (lane / (8 * F)) * run;
+  const int px = c & 1, py = 2 + ((c >> 1) & 1), pz = 4 + (c >> 2);
+  const int64_t left = n - i0;
+  const int steps = left < run ? (int)left : run;  // points past n hold zero gradients
   float* gtab = grad + (size_t)p.off * F + f;
-  uint32_t id[8];
-  float w[8];
-  cell_corners(cell, p, id);
-  cell_weights(t, w);
-#pragma unroll
-  for (int c = 0; c < 8; ++c) atomic_add_f32(gtab + (size_t)id[c] * F, w[c] * g);
+  float acc = 0.0f;
+  uint32_t cur = 0xffffffffu;
+#pragma unroll 4
+  for (int s = 0; s < steps; ++s) {
+    const float g = s_g[wave][first + s][f];
+    if (g == 0.0f) continue;  // adding +0 leaves the accumulator unchanged
+    const float2 ax = s_axis[wave][first + s][px], ay = s_axis[wave][first + s][py],
+                 az = s_axis[wave][first + s][pz];
+    const uint32_t tx = __float_as_uint(ax.y), ty = __float_as_uint(ay.y),
+                   tz = __float_as_uint(az.y);
+    uint32_t id;
+    if (p.hashed) {
+      id = (tx ^ ty ^ tz) & (p.size - 1u);
+    } else {
+      id = tx + ty + tz;
+      if (__builtin_expect(id >= p.size, 0)) id %= p.size;
+    }
+    const float w = ax.x * ay.x * az.x;
+    if (id != cur) {
+      if (acc != 0.0f) atomic_add_f32(gtab + (size_t)cur * F, acc);
+      cur = id;
+      acc = 0.0f;
+    }
+    acc = fmaf(w, g, acc);
+  }
+  if (acc != 0.0f) atomic_add_f32(gtab + (size_t)cur * F, acc);
 }
 
 constexpr float kTapDir[4][3] = {{1, -1, -1}, {-1, -1, 1}, {-1, 1, -1}, {1, 1, 1}};
@@ -965,10 +1040,17 @@ struct BwdLaunch {
 template <int F, typename TD>
 static int launch_bwd(const BwdLaunch& a) {
   if (a.active <= 0) return NA_OK;
+  // points per wave: whole 64-point batches, fewer where those would leave most
+  // of the chip's wave slots empty
+  int run = 8 * F;
+  while (run > 8 && ceil_div(a.n, (int64_t)(64 / (8 * F)) * run) * a.active < 8192) run /= 2;
+  const int64_t per_block = (int64_t)kBwdWaves * (64 / (8 * F)) * run;
   dim3 grid;
-  if (int st = chunk_level_grid(ceil_div(a.n * F, kBlock), a.active, &grid)) return st;
+  if (int st = chunk_level_grid(ceil_div(a.n, per_block), a.active, &grid)) return st;
+  constexpr size_t kAlign = F * sizeof(TD) < 16 ? F * sizeof(TD) : 16;  // of the vector loads
+  const int vec = ((uintptr_t)a.dy % kAlign) == 0 && (a.ld * sizeof(TD)) % kAlign == 0;
   hipLaunchKernelGGL((hashgrid_bwd_kernel<F, TD>), grid, dim3(kBlock), 0, a.s, *a.d, a.x, a.n,
-                     a.vmin, a.vrange, (const TD*)a.dy, a.ld, a.grad, a.active);
+                     a.vmin, a.vrange, (const TD*)a.dy, a.ld, vec, a.grad, a.active, run);
   NA_CHECK_LAUNCH();
   return NA_OK;
 }
