@@ -148,15 +148,11 @@ __device__ inline void epilogue_store(const EpiParams& e, int64_t m, int64_t n, 
   }
 }
 
-// Per element type: K-tile depth, LDS row pitch (elements) and MFMA step.
-//   bf16: BK = 32, pitch 40 (80 B rows keep 16-byte MFMA operand reads aligned)
-//   fp32: BK = 16, pitch 17 (odd pitch: conflict-free single-float operand reads)
+// K-tile depth and LDS row pitch (elements) of the general bf16 kernel: 80-byte
+// rows keep its 16-byte MFMA operand reads aligned.
 template <typename T> struct GemmCfg;
 template <> struct GemmCfg<bf16_t> {
   static constexpr int BK = 32, LDK = 40;
-};
-template <> struct GemmCfg<float> {
-  static constexpr int BK = 16, LDK = 17;
 };
 
 // Global -> register stage of one [128 x BK] operand tile, then register -> LDS
@@ -174,7 +170,7 @@ struct TileLoader {
     uint4 q;
     T e[VEC];
   };
-  static_assert(sizeof(T) != 2 || NVEC == 2, "bf16 transposed loads pair two k rows");
+  static_assert(sizeof(T) == 2 && NVEC == 2, "transposed loads pair two k rows");
   Vec reg[NVEC];
 
   __device__ inline void load(const T* __restrict__ X, int64_t ld, int64_t r0, int64_t rmax,
@@ -190,19 +186,9 @@ struct TileLoader {
         } else {
           reg[j].q = make_uint4(0, 0, 0, 0);
         }
-      } else if constexpr (sizeof(T) == 2) {
-        // bf16: thread t owns rows 8*(t%16)..+7 at k = 2*(t/16) + j
-        const int r = (tid % (GBM / VEC)) * VEC, k = 2 * (tid / (GBM / VEC)) + j;
-        const int64_t gr = r0 + r, gk = k0 + k;
-        if (gk < kend && gr + VEC <= rmax) {
-          reg[j].q = *reinterpret_cast<const uint4*>(X + gk * ld + gr);
-        } else {
-#pragma unroll
-          for (int e = 0; e < VEC; ++e)
-            reg[j].e[e] = (gk < kend && gr + e < rmax) ? X[gk * ld + gr + e] : T(0);
-        }
       } else {
-        const int k = v / (GBM / VEC), r = (v % (GBM / VEC)) * VEC;
+        // thread t owns rows 8*(t%16)..+7 at k = 2*(t/16) + j
+        const int r = (tid % (GBM / VEC)) * VEC, k = 2 * (tid / (GBM / VEC)) + j;
         const int64_t gr = r0 + r, gk = k0 + k;
         if (gk < kend && gr + VEC <= rmax) {
           reg[j].q = *reinterpret_cast<const uint4*>(X + gk * ld + gr);
@@ -221,13 +207,8 @@ struct TileLoader {
       const int v = j * GNT + tid;
       if (!TRANS) {
         const int r = v / (BK / VEC), k = (v % (BK / VEC)) * VEC;
-        if constexpr (sizeof(T) == 2) {
-          *reinterpret_cast<uint4*>(s + r * LDK + k) = reg[j].q;
-        } else {
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) s[r * LDK + k + e] = reg[j].e[e];
-        }
-      } else if constexpr (sizeof(T) == 2) {
+        *reinterpret_cast<uint4*>(s + r * LDK + k) = reg[j].q;
+      } else {
         // transpose the thread's 2 (k) x 8 (r) block in registers: one 32-bit
         // LDS store per row holds the (k, k+1) pair
         if (j == 0) {
@@ -242,10 +223,6 @@ struct TileLoader {
             *reinterpret_cast<uint32_t*>(s + (r + 2 * e + 1) * LDK + k) = hi;
           }
         }
-      } else {
-        const int k = v / (GBM / VEC), r = (v % (GBM / VEC)) * VEC;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) s[(r + e) * LDK + k] = reg[j].e[e];
       }
     }
   }
@@ -274,31 +251,6 @@ template <> struct MfmaStep<bf16_t> {
     }
   }
 };
-template <> struct MfmaStep<float> {
-  static constexpr int LDK = GemmCfg<float>::LDK;
-  __device__ static inline void run(const float* As, const float* Bs, int wm, int wn, int lane,
-                                    f32x16_t acc[2][2]) {
-#pragma unroll
-    for (int kk = 0; kk < GemmCfg<float>::BK; kk += 2) {
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = As[(wm * 64 + i * 32 + (lane & 31)) * LDK + kk + (lane >> 5)];
-        b[i] = Bs[(wn * 64 + i * 32 + (lane & 31)) * LDK + kk + (lane >> 5)];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-  }
-};
-
-// Epilogue shared by the GEMM kernels: per half (i), each wave stages a 32 x 64
-// accumulator block through LDS (`smem`, at least 4*32*65 floats, free to
-// reuse) so that every accumulator register is addressed statically and the
-// global stores run along rows (64 consecutive columns per wave instruction).
 // Epilogue shared by the GEMM kernels: per half (i), each wave stages a 32 x 64
 // accumulator block through LDS (`smem`, at least 4*32*65 floats, free to
 // reuse) so that every accumulator register is addressed statically and the
@@ -315,9 +267,10 @@ __device__ __attribute__((always_inline)) inline float epi_row_operand(const Epi
   return 0.0f;
 }
 
-template <int RB, bool PIPE>
+// NI: 32-row blocks per wave.
+template <int RB, bool PIPE, int NI>
 __device__ __attribute__((always_inline)) inline void gemm_epilogue(
-    const GemmParams& p, unsigned char* smem, f32x16_t (&acc)[2][2], int64_t m0, int64_t n0,
+    const GemmParams& p, unsigned char* smem, f32x16_t (&acc)[NI][2], int64_t m0, int64_t n0,
     int wm, int wn, int wave, int lane) {
   constexpr int CP = 65;
   float* Cw = reinterpret_cast<float*>(smem) + wave * 32 * CP;
@@ -326,15 +279,15 @@ __device__ __attribute__((always_inline)) inline void gemm_epilogue(
   const bool ncol = n < p.N;
   const bool head = e.head_w != nullptr;
   const bool rowop = PIPE && (e.zc || e.dact);
-  const int64_t part = 2 * (2 * (int64_t)blockIdx.y + wn);  // first of the wave's two 32-column parts
+  const int64_t part = 2 * (n0 / 64 + wn);  // first of the wave's two 32-column parts
   // per-column operands, loaded once
   const float hw = (head && ncol) ? e.head_w[n] : 0.0f;
   const float bias_n = (e.bias && ncol) ? e.bias[n] : 0.0f;
   const float r1b_n = (e.r1_a && ncol) ? e.r1_b[n] : 0.0f;
   float csum = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int64_t mb = m0 + wm * 64 + i * 32;
+  for (int i = 0; i < NI; ++i) {
+    const int64_t mb = m0 + (wm * NI + i) * 32;
     float nxt[RB];
 #pragma unroll
     for (int u = 0; u < RB; ++u) nxt[u] = rowop ? epi_row_operand(e, mb + u, n, ncol && mb + u < p.M) : 0.0f;
@@ -1812,6 +1765,356 @@ gemm_bf16_nn_persist_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// float32 GEMM on the bf16 matrix cores.
+//
+// A float32 value is the exact sum of three bf16 values, x = x1 + x2 + x3 (x1 =
+// bf16(x), x2 = bf16(x - x1), x3 = the rest: 3 x 8 significand bits), so a
+// product is x y = x1 y1 + (x1 y2 + x2 y1) + (x2 y2 + x1 y3 + x3 y1) up to terms of
+// 2^-25 |x y| and below, under the rounding of one float32 multiply.  A 16-wide
+// step of the bf16 instruction six times takes 192 cycles where the float32
+// instruction takes 512.  x1 y1 and the five smaller products have accumulators of
+// their own: the instruction drops the bits that fall below the sum it adds to
+// (always downwards), which six additions a step into one sum turned into a bias
+// of 1.2e-8 of the result; apart, the bias is 2e-10 and the error against float64
+// 0.67e-7 at K = 136 and 0.9e-7 at K = 256, where the float32 instruction's is
+// 2.1e-7 and 2.9e-7 (normally distributed operands).
+// A value that is not finite, or whose x1 rounds to infinity (3.39e38 and above),
+// leaves infinities or NaN in the accumulators of its rows or columns: a wave that
+// ends with one forms its tile again on the float32 instruction, so such values come out
+// as they do there.
+//
+// A workgroup covers 128 rows x up to 128 columns (160 where one tile holds all),
+// 32 rows per wave; the whole 256 columns of a layer in one tile would split the A rows
+// once, but the accumulators of both kinds do not fit the registers of two waves per SIMD.
+// Per 32-wide K stage a thread reads float32 chunks one stage ahead, splits them and
+// writes 16-byte chunks of the three bf16 planes to LDS (XOR-swizzled,
+// conflict-free); two workgroups per CU overlap each other's barriers.
+// Rows x columns x K, float32 instruction -> here: 2,146,689 x 256 x 136 2.18 -> 1.43 ms,
+// 98,304 x 256 x 280 168 -> 95 us, 49,152 x 256 x 256 84 -> 53 us, 4,096 x 256 x 68 28 -> 8 us;
+// transposed (weight gradients; before, also too few parts of the sum): 256 x 136 over
+// 196,608 rows 427 -> 162 us, 256 x 280 over 28,800 rows 302 -> 58 us, 256 x 84 over 3,200
+// rows 380 -> 14 us.
+typedef __attribute__((ext_vector_type(8))) float f32x8_t;
+
+__device__ inline void split3(const f32x8_t& x, bf16x8_t (&h)[3]) {
+  h[0] = __builtin_convertvector(x, bf16x8_t);
+  const f32x8_t r = x - __builtin_convertvector(h[0], f32x8_t);
+  h[1] = __builtin_convertvector(r, bf16x8_t);
+  h[2] = __builtin_convertvector(r - __builtin_convertvector(h[1], f32x8_t), bf16x8_t);
+}
+
+constexpr int kF3BK = 32, kF3BM = 128;
+
+// One operand tile of R rows x 32 k, float32 chunks in registers.  Rows past the
+// operand's end repeat its last ones: they only reach outputs that are not stored.
+// load() issues the stage's loads and nothing else, so they stay in flight during the
+// products; what lies past the end of K is cleared by store().
+// TRANS = false: element (r, k) at X[r ld + k], a thread takes 8 k of NC rows, 64 apart.
+// TRANS = true: element (r, k) at X[k ld + r], threads t < R take 4 r x 8 k each (NC = 4);
+// QUADS: the operand's width is a multiple of 4 (else element by element).
+template <int NC, int R, bool TRANS, bool QUADS>
+struct SplitLoader {
+  float4 q[NC][2];  // TRANS: k row e of the thread's 8 at q[e / 2][e % 2]
+  const float* row[TRANS ? 1 : NC];
+  int64_t left;  // TRANS: rows from the thread's first to the operand's end
+
+  __device__ inline void init(const float* __restrict__ X, int64_t ld, int64_t r0, int64_t rmax,
+                              int64_t kbeg, int t) {
+    if constexpr (!TRANS) {
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        const int64_t r = r0 + (j * GNT + t) / 4;
+        row[j] = X + (r < rmax ? r : rmax - 1) * ld + kbeg;
+      }
+    } else {
+      int64_t r = r0 + t % (R / 4) * 4;
+      if (QUADS && r >= rmax) r = rmax - 4;
+      left = rmax - r;
+      row[0] = X + kbeg * ld + r;
+    }
+  }
+
+  __device__ static inline int first_k(int t) {
+    return TRANS ? (t < R ? t / (R / 4) * 8 : 0) : (t & 3) * 8;
+  }
+
+  // the stage at k offset `k` from kbeg with `n` > 0 values of k left (32 or more: a whole
+  // stage); k past the end reads the stage's first place instead
+  __device__ inline void load(int64_t ld, int64_t k, int64_t n, int t) {
+    const int c = first_k(t);
+    if constexpr (!TRANS) {
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          q[j][e] = *reinterpret_cast<const float4*>(row[j] + k + (c + 4 * e < n ? c + 4 * e : 0));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float* s = row[0] + (k + (c + e < n ? c + e : 0)) * ld;
+        if constexpr (QUADS) {
+          q[e / 2][e % 2] = *reinterpret_cast<const float4*>(s);
+        } else {
+          q[e / 2][e % 2] = make_float4(left > 0 ? s[0] : 0.0f, left > 1 ? s[1] : 0.0f,
+                                        left > 2 ? s[2] : 0.0f, left > 3 ? s[3] : 0.0f);
+        }
+      }
+    }
+  }
+
+  __device__ inline void store(bf16_t* __restrict__ planes, int64_t n, int t) {
+    if (TRANS && t >= R) return;
+    const int c = first_k(t);
+    if (n < kF3BK) {
+      const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (c + (TRANS ? 2 * j + e : 4 * e) >= n) q[j][e] = zero;
+    }
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int r = TRANS ? t % (R / 4) * 4 + j : (j * GNT + t) / 4;
+      if (!TRANS && r >= R) continue;
+      f32x8_t x;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float4 u = TRANS ? q[e / 2][e % 2] : q[j][e / 4];
+        const int i = TRANS ? j : e % 4;
+        x[e] = i == 0 ? u.x : (i == 1 ? u.y : (i == 2 ? u.z : u.w));
+      }
+      bf16x8_t h[3];
+      split3(x, h);
+      bf16_t* d = planes + r * kF3BK + (((c >> 3) ^ ((r >> 2) & 3)) << 3);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8_t*>(d + k * R * kF3BK) = h[k];
+    }
+  }
+};
+
+// element (r, k) of an operand, zero outside it
+template <bool TRANS>
+__device__ inline float f3_at(const float* __restrict__ X, int64_t ld, int64_t r, int64_t rmax,
+                              int64_t k, int64_t kend) {
+  if (r >= rmax || k >= kend) return 0.0f;
+  return TRANS ? X[k * ld + r] : X[r * ld + k];
+}
+
+// Where the outputs go.  F3_ROWS: a lane holds 16 columns of one row per 32 x 32 block
+// (the weights are the first MFMA operand) and finishes them in registers, 8 at a
+// time, with 16-byte loads and stores.  F3_ATOMIC: a lane holds one column (rows in
+// registers), so an atomic instruction covers whole row segments.  F3_GENERAL: the
+// staged epilogue, for unaligned rows, widths that are not multiples of 8 and the
+// rare epilogue terms.
+enum F3Mode : int { F3_ROWS, F3_ATOMIC, F3_GENERAL };
+
+__device__ inline float sum_lanes32(float v) {  // over the lanes that share lane >> 5
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, false));
+  return v + __shfl_xor(v, 16);
+}
+
+// eight columns of one row: bias, activation, rank-1 term, derivative of the stored activation
+__device__ inline void f3_finish8(const EpiParams& e, int64_t m, int64_t col, float r1, float (&v)[8]) {
+  if (e.bias) {
+    float b[8];
+    vload8(e.bias + col, b);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] += b[c];
+  }
+  if (e.act == NA_ACT_RELU) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = v[c] > 0.0f ? v[c] : 0.0f;
+  } else if (e.act == NA_ACT_SOFTPLUS) {
+    const float ib = 1.0f / e.beta;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = softplus_sel(v[c], e.beta, ib);
+  } else if (e.act) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = act_forward(e.act, v[c], e.beta);
+  }
+  if (e.r1_a) {
+    float b[8];
+    vload8(e.r1_b + col, b);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] += r1 * b[c];
+  }
+  if (e.dact) {
+    float y[8];
+    if (e.dact_dtype == NA_BF16) vload8((const bf16_t*)e.dact_y + m * e.ld_dact + col, y);
+    else vload8((const float*)e.dact_y + m * e.ld_dact + col, y);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] *= act_deriv_from_y(e.dact, y[c], e.beta);
+  }
+}
+
+template <bool TA, bool TB, int NB, int MODE>
+__global__ void __launch_bounds__(GNT, 2)
+gemm_f32_kernel(GemmParams p, int64_t parts) {
+  constexpr int BM = kF3BM, BN = 32 * NB;
+  constexpr int PLANES = 3 * (BM + BN) * kF3BK * 2;
+  constexpr int STAGED = MODE == F3_GENERAL ? 4 * 32 * 65 * 4 : BN * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[PLANES > STAGED ? PLANES : STAGED];
+  bf16_t* Ap = reinterpret_cast<bf16_t*>(smem);
+  bf16_t* Bp = Ap + 3 * BM * kF3BK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // a unit is a row tile of one part of K; its column tiles share the A rows and run back
+  // to back on one XCD (few units: in plain order, so that all XCDs take part)
+  const uint32_t ncol = (uint32_t)((p.N + BN - 1) / BN), slot = blockIdx.x >> 3;
+  const int64_t rows = (p.M + BM - 1) / BM, units = rows * parts;
+  const int64_t unit = units < 64 ? blockIdx.x / ncol : (int64_t)(slot / ncol) * 8 + (blockIdx.x & 7);
+  if (unit >= units) return;
+  const int64_t m0 = unit % rows * BM;
+  const int64_t n0 = (int64_t)((units < 64 ? blockIdx.x : slot) % ncol) * BN;
+  const int64_t kbeg = unit / rows * p.k_chunk;
+  const int64_t kend = kbeg + p.k_chunk < p.K ? kbeg + p.k_chunk : p.K;
+
+  f32x16_t acc[NB], low[NB];  // x1 y1, and the five smaller products
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = low[j][r] = 0.0f;
+
+  SplitLoader<TA ? 4 : BM / 64, BM, TA, MODE != F3_GENERAL> la;
+  SplitLoader<TB ? 4 : (BN + 63) / 64, BN, TB, MODE != F3_GENERAL> lb;
+  // transposed tiles of 128 rows and up to 128 columns use one half of the threads each
+  const int tb = TA && TB ? (tid + GNT / 2) & (GNT - 1) : tid;
+  la.init((const float*)p.A, p.lda, m0, p.M, kbeg, tid);
+  lb.init((const float*)p.B, p.ldb, n0, p.N, kbeg, tb);
+  if (kbeg < kend) {
+    la.load(p.lda, 0, kend - kbeg, tid);
+    lb.load(p.ldb, 0, kend - kbeg, tb);
+  }
+  for (int64_t k0 = kbeg; k0 < kend; k0 += kF3BK) {
+    la.store(Ap, kend - k0, tid);
+    lb.store(Bp, kend - k0, tb);
+    __syncthreads();
+    if (k0 + kF3BK < kend) {
+      la.load(p.lda, k0 + kF3BK - kbeg, kend - k0 - kF3BK, tid);
+      lb.load(p.ldb, k0 + kF3BK - kbeg, kend - k0 - kF3BK, tb);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      if (kk == 1 && kend - k0 <= 16) break;  // the last stage's second half is empty
+      const int ck = 2 * kk + (lane >> 5);
+      constexpr int kTerms[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+      bf16x8_t a[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int r = wave * 32 + (lane & 31);
+        a[q] = *reinterpret_cast<const bf16x8_t*>(Ap + (q * BM + r) * kF3BK + ((ck ^ ((r >> 2) & 3)) << 3));
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        bf16x8_t b[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const int r = j * 32 + (lane & 31);
+          b[q] = *reinterpret_cast<const bf16x8_t*>(Bp + (q * BN + r) * kF3BK + ((ck ^ ((r >> 2) & 3)) << 3));
+        }
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+          const bf16x8_t &x = a[kTerms[t][0]], &y = b[kTerms[t][1]];
+          f32x16_t& d = t < 5 ? low[j] : acc[j];
+          d = MODE == F3_ROWS ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(y, x, d, 0, 0, 0)
+                              : __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, d, 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  bool fine = true;
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc[j][r] += low[j][r];
+      fine = fine && fabsf(acc[j][r]) < INFINITY;
+    }
+  if (__builtin_expect(__any(!fine), 0)) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+#pragma unroll 1
+    for (int64_t k = kbeg + (lane >> 5); k < kend + (lane >> 5); k += 2) {
+      const float x = f3_at<TA>((const float*)p.A, p.lda, m0 + wave * 32 + (lane & 31), p.M, k, kend);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const float y = f3_at<TB>((const float*)p.B, p.ldb, n0 + j * 32 + (lane & 31), p.N, k, kend);
+        acc[j] = MODE == F3_ROWS ? __builtin_amdgcn_mfma_f32_32x32x2f32(y, x, acc[j], 0, 0, 0)
+                                 : __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[j], 0, 0, 0);
+      }
+    }
+  }
+
+  if constexpr (MODE == F3_ATOMIC) {
+    float* C = (float*)p.e.C;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int64_t n = n0 + j * 32 + (lane & 31);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t m = m0 + wave * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (m < p.M && n < p.N) atomic_add_f32(C + m * p.e.ldc + n, acc[j][r]);
+      }
+    }
+  } else if constexpr (MODE == F3_ROWS) {
+    const EpiParams& e = p.e;
+    const int64_t m = m0 + wave * 32 + (lane & 31);
+    const bool in = m < p.M;
+    const float r1 = e.r1_a && in ? e.r1_a[m] : 0.0f;
+    float* s_col = reinterpret_cast<float*>(smem);  // the last barrier freed the planes
+    if (e.colsum) {
+      for (int c = tid; c < BN; c += GNT) s_col[c] = 0.0f;
+      __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int gq = 0; gq < 2; ++gq) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[j][8 * gq + q]),
+                                                          __float_as_uint(acc[j][8 * gq + 4 + q]), false, false);
+          v[q] = __uint_as_float(r[0]);
+          v[4 + q] = __uint_as_float(r[1]);
+        }
+        const int64_t col = n0 + 32 * j + 16 * gq + 8 * (lane >> 5);
+        const bool ok = in && col < p.N;
+        if (ok) {
+          f3_finish8(e, m, col, r1, v);
+          if (e.c_dtype == NA_BF16) vstore8((bf16_t*)e.C + m * e.ldc + col, v);
+          else vstore8((float*)e.C + m * e.ldc + col, v);
+        }
+        if (e.colsum) {
+#pragma unroll
+          for (int c = 0; c < 8; ++c) {
+            const float t = sum_lanes32(ok ? v[c] : 0.0f);
+            if ((lane & 31) == 0) atomicAdd(s_col + (col - n0) + c, t);
+          }
+        }
+      }
+    if (e.colsum) {
+      __syncthreads();
+      for (int c = tid; c < BN; c += GNT)
+        if (n0 + c < p.N) atomic_add_f32(e.colsum + n0 + c, s_col[c]);
+    }
+  } else {
+    static_assert(MODE != F3_GENERAL || NB == 4, "the staged epilogue takes 64 columns at a time");
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      f32x16_t part[1][2] = {{acc[2 * half], acc[2 * half + 1]}};
+      gemm_epilogue<4, false>(p, smem, part, m0, n0, wave, half, wave, lane);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Weights-stationary GEMM for the 256-wide MLP layers: C = epi(A . B^T) with
 // N = 256, M a multiple of 128 and NK 32-wide K stages.  Eight waves each own
 // 32 output columns and hold those columns' weights over the whole K range in
@@ -2758,24 +3061,95 @@ static int launch_wgrad(const na_gemm_args* a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-template <typename T>
-static int launch_gemm(const na_gemm_args* a, const GemmParams& p, dim3 grid, hipStream_t s) {
-  if (!a->trans_a && !a->trans_b) {
-    if constexpr (sizeof(T) == 2)
-      hipLaunchKernelGGL(gemm_bf16_nn_kernel, grid, dim3(GNT), 0, s, p);
-    else
-      hipLaunchKernelGGL((gemm_kernel<T, false, false>), grid, dim3(GNT), 0, s, p);
-  }
+static int launch_gemm_bf16(const na_gemm_args* a, const GemmParams& p, dim3 grid, hipStream_t s) {
+  if (!a->trans_a && !a->trans_b)
+    hipLaunchKernelGGL(gemm_bf16_nn_kernel, grid, dim3(GNT), 0, s, p);
   else if (!a->trans_a && a->trans_b)
-    hipLaunchKernelGGL((gemm_kernel<T, false, true>), grid, dim3(GNT), 0, s, p);
+    hipLaunchKernelGGL((gemm_kernel<bf16_t, false, true>), grid, dim3(GNT), 0, s, p);
   else if (a->trans_a && a->trans_b)
-    hipLaunchKernelGGL((gemm_kernel<T, true, true>), grid, dim3(GNT), 0, s, p);
+    hipLaunchKernelGGL((gemm_kernel<bf16_t, true, true>), grid, dim3(GNT), 0, s, p);
   else
-    hipLaunchKernelGGL((gemm_kernel<T, true, false>), grid, dim3(GNT), 0, s, p);
+    hipLaunchKernelGGL((gemm_kernel<bf16_t, true, false>), grid, dim3(GNT), 0, s, p);
   NA_CHECK_LAUNCH();
   return NA_OK;
 }
 
+// Rows that F3_ROWS stores and loads 8 at a time.
+static bool f32_rows_ok(const na_gemm_args* a) {
+  auto rows8 = [](const void* p, int64_t ld, int dtype) {
+    return aligned16(p) && (ld * (dtype == NA_BF16 ? 2 : 4)) % 16 == 0;
+  };
+  return a->epilogue == NA_EPI_STORE && a->N % 8 == 0 && rows8(a->C, a->ldc, a->c_dtype) &&
+         !a->z_out && !a->zc && !a->head_w && (!a->bias || aligned16(a->bias)) &&
+         (!a->r1_a || aligned16(a->r1_b)) && (!a->dact || rows8(a->dact_y, a->ld_dact, a->dact_dtype));
+}
+
+template <bool TA, bool TB, int MODE>
+static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
+  // Split the sum over K where the output is added with atomics and no epilogue term
+  // is nonlinear: two workgroups per CU, of at least 96 values each.  (The weight
+  // gradients ask for a part per 2048 rows, which leaves most CUs idle below half
+  // a million rows: 380 us at 3,200 rows, where 34 parts take 14.)
+  const int64_t rows = ceil_div(p.M, (int64_t)kF3BM), blocks = ceil_div(p.N, (int64_t)32);
+  int64_t cols = blocks <= 5 ? 1 : ceil_div(blocks, (int64_t)4), parts = 1;
+  if (MODE == F3_GENERAL) {
+    cols = ceil_div(blocks, (int64_t)4);
+    if (a->split_k > 1) parts = a->split_k;
+  } else if (MODE == F3_ATOMIC) {
+    // transposed tiles of up to 96 columns load beside the 128 rows, with both
+    // accumulators in registers
+    cols = ceil_div(blocks, (int64_t)3);
+    const int64_t most = ceil_div(p.K, (int64_t)96);
+    parts = ceil_div((int64_t)512, rows * cols);
+    if (parts > most) parts = most;
+  } else {
+    // narrower tiles where these would leave CUs idle
+    while (rows * cols < 512 && cols * 2 <= blocks) cols *= 2;
+  }
+  int nb = MODE == F3_GENERAL ? 4 : (int)ceil_div(blocks, cols);
+  cols = ceil_div(blocks, (int64_t)nb);
+  p.k_chunk = ceil_div(ceil_div(p.K, parts < 1 ? 1 : parts), (int64_t)kF3BK) * kF3BK;
+  if (p.k_chunk < kF3BK) p.k_chunk = kF3BK;
+  parts = p.K == 0 ? 1 : ceil_div(p.K, p.k_chunk);
+  const int64_t units = rows * parts;
+  const int64_t blocks_all = units < 64 ? units * cols : ceil_div(units, (int64_t)8) * 8 * cols;
+  NA_CHECK_ARG(blocks_all < 0x7fffffffLL, "GEMM grid too large");
+  const dim3 grid((unsigned)blocks_all);
+#define NA_F3(NB) hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, NB, MODE>), grid, dim3(GNT), 0, s, p, parts)
+  if constexpr (MODE == F3_GENERAL) {
+    NA_F3(4);
+  } else if constexpr (MODE == F3_ATOMIC) {
+    switch (nb) {
+      case 1: NA_F3(1); break;
+      case 2: NA_F3(2); break;
+      default: NA_F3(3); break;
+    }
+  } else {
+    switch (nb) {
+      case 1: NA_F3(1); break;
+      case 2: NA_F3(2); break;
+      case 3: NA_F3(3); break;
+      case 4: NA_F3(4); break;
+      default: NA_F3(5); break;
+    }
+  }
+#undef NA_F3
+  NA_CHECK_LAUNCH();
+  return NA_OK;
+}
+
+static int run_gemm_f32(const na_gemm_args* a, const GemmParams& p, hipStream_t s) {
+  if (a->trans_a && a->trans_b) {
+    const bool plain = a->epilogue == NA_EPI_ATOMIC && !a->bias && !a->act && !a->dact && !a->r1_a &&
+                       !a->colsum && a->M % 4 == 0 && a->N % 4 == 0;
+    return plain ? launch_gemm_f32<true, true, F3_ATOMIC>(a, p, s)
+                 : launch_gemm_f32<true, true, F3_GENERAL>(a, p, s);
+  }
+  if (a->trans_a) return launch_gemm_f32<true, false, F3_GENERAL>(a, p, s);
+  if (a->trans_b) return launch_gemm_f32<false, true, F3_GENERAL>(a, p, s);
+  return f32_rows_ok(a) ? launch_gemm_f32<false, false, F3_ROWS>(a, p, s)
+                        : launch_gemm_f32<false, false, F3_GENERAL>(a, p, s);
+}
 
 // Vectorised act_grad for rows of whole 16-byte chunks (N a multiple of 8 with
 // N / 8 dividing 256): thread (r, c) of a block handles columns 8 c .. 8 c + 7
@@ -3036,7 +3410,7 @@ extern "C" int na_gemm(const na_gemm_args* a, na_stream_t stream) {
   GemmParams p;
   p.M = a->M; p.N = a->N; p.K = a->K;
   p.A = a->A; p.lda = a->lda; p.B = a->B; p.ldb = a->ldb;
-  const int64_t bk = a->in_dtype == NA_BF16 ? GemmCfg<bf16_t>::BK : GemmCfg<float>::BK;
+  const int64_t bk = GemmCfg<bf16_t>::BK;
   int64_t kc = ceil_div(ceil_div(a->K, split), bk) * bk;
   if (kc < bk) kc = bk;
   p.k_chunk = kc;
@@ -3073,8 +3447,8 @@ extern "C" int na_gemm(const na_gemm_args* a, na_stream_t stream) {
       return NA_OK;
     }
   }
-  if (a->in_dtype == NA_BF16) return launch_gemm<bf16_t>(a, p, grid, s);
-  return launch_gemm<float>(a, p, grid, s);
+  if (a->in_dtype == NA_BF16) return launch_gemm_bf16(a, p, grid, s);
+  return run_gemm_f32(a, p, s);
 }
 
 static bool narrow_vec_ok(int64_t K, int64_t ld, const void* X, int dtype) {

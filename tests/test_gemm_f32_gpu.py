@@ -1,0 +1,89 @@
+"""The float32 products at tile, stage and split edges, in every operand layout, against
+float64; and with values that do not split into bf16 parts."""
+import pytest
+import torch
+
+from neuralangelo_amd import functional as Fn
+from neuralangelo_amd._lib import NA_ACT_RELU, NA_ACT_SOFTPLUS, NA_EPI_ATOMIC, NA_EPI_STORE
+
+pytestmark = pytest.mark.gpu
+
+
+def operand(rows, k, trans, g, scale=1.0):
+    """[rows, k] values and their storage ([rows, ld] or, transposed, [k, ld]; ld % 4 == 0)."""
+    v = (torch.randn(rows, k, generator=g) * scale).cuda()
+    m = v.t() if trans else v
+    ld = (m.shape[1] + 3) // 4 * 4
+    s = torch.full((m.shape[0], ld), 7.0, device="cuda")  # the padding is never part of a product
+    s[:, :m.shape[1]] = m
+    return v, s, ld
+
+
+def bound(A, B, k):
+    """One rounding per product and one per addition, in any order."""
+    return (k + 16) * 2.0 ** -24 * (A.double().abs() @ B.double().abs().t()) + 1e-37
+
+
+@pytest.mark.parametrize("ta, tb", [(0, 0), (1, 1), (1, 0), (0, 1)])
+@pytest.mark.parametrize("M, N, K", [(1, 8, 4), (127, 256, 68), (128, 136, 136), (131, 280, 256),
+                                     (70, 3, 20), (257, 160, 100), (4100, 96, 36), (64, 84, 3204)])
+def test_layouts_and_edges(M, N, K, ta, tb):
+    g = torch.Generator().manual_seed(M + N + K)
+    A, a, lda = operand(M, K, ta, g)
+    B, b, ldb = operand(N, K, tb, g)
+    ref = A.double() @ B.double().t()
+    C = torch.full((M, N), 3.0, device="cuda")
+    Fn.gemm(a, lda, ta, b, ldb, tb, M, N, K, C, N)
+    assert ((C.double() - ref).abs() <= bound(A, B, K)).all()
+    C.fill_(0.5)
+    Fn.gemm(a, lda, ta, b, ldb, tb, M, N, K, C, N, epilogue=NA_EPI_ATOMIC, split_k=3)
+    # each part's sum is rounded once more as it is added
+    parts = -(-K // 32)
+    slack = (parts + 2) * 2.0 ** -24 * (ref.abs() + 0.5 + (A.double().abs() @ B.double().abs().t()))
+    assert ((C.double() - ref - 0.5).abs() <= bound(A, B, K) + slack).all()
+
+
+@pytest.mark.parametrize("M, N, K", [(5, 8, 16), (129, 256, 68), (640, 272, 256)])
+def test_epilogue_terms(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    A, a, lda = operand(M, K, 0, g, 0.1)
+    B, b, ldb = operand(N, K, 0, g, 0.1)
+    bias = torch.randn(N, generator=g).cuda()
+    z = A.double() @ B.double().t() + bias.double()
+    err = bound(A, B, K) + 2.0 ** -23 * z.abs()
+    for act, ref in ((NA_ACT_RELU, z.relu()), (NA_ACT_SOFTPLUS, torch.nn.functional.softplus(z, beta=100))):
+        C = torch.empty(M, N, device="cuda")
+        Fn.gemm(a, lda, 0, b, ldb, 0, M, N, K, C, N, bias=bias, act=act)
+        # both have slopes of at most 1; softplus adds a few ulps of 1 / beta
+        assert ((C.double() - ref).abs() <= err + 1e-8 + 2.0 ** -22 * ref.abs()).all()
+    y = torch.rand(M, N, generator=g).cuda() - 0.3
+    r1a, r1b = torch.randn(M, generator=g).cuda(), torch.randn(N, generator=g).cuda()
+    C, cs = torch.empty(M, N, device="cuda"), torch.ones(N, device="cuda")
+    Fn.gemm(a, lda, 0, b, ldb, 0, M, N, K, C, N, dact=NA_ACT_RELU, dact_y=y, ld_dact=N, r1_a=r1a,
+            r1_b=r1b, colsum=cs)
+    v = (z - bias.double() + r1a.double()[:, None] * r1b.double()) * (y > 0)
+    e = err + 2.0 ** -22 * (r1a.double()[:, None] * r1b.double()).abs()
+    assert ((C.double() - v).abs() <= e).all()
+    assert ((cs.double() - 1 - v.sum(0)).abs() <= e.sum(0) + M * 2.0 ** -23 * (1 + v.abs().sum(0))).all()
+
+
+@pytest.mark.parametrize("ta, tb, N", [(0, 0, 264), (1, 1, 64), (0, 0, 5)])
+def test_values_that_do_not_split(ta, tb, N):
+    M, K = 300, 64
+    g = torch.Generator().manual_seed(N)
+    A, a, lda = operand(M, K, ta, g)
+    B, b, ldb = operand(N, K, tb, g, 1e-3)
+    sa, sb = (a.t() if ta else a), (b.t() if tb else b)
+    for m, k, v in ((3, 5, float("inf")), (40, 0, float("nan")), (200, 63, 3.4e38), (299, 7, -float("inf"))):
+        A[m, k] = sa[m, k] = v
+    B[2, 9] = sb[2, 9] = -3.4e38
+    B[4, 11] = sb[4, 11] = 0.0
+    ref = A.double() @ B.double().t()
+    C = torch.zeros(M, N, device="cuda")
+    epi = NA_EPI_ATOMIC if ta else NA_EPI_STORE
+    Fn.gemm(a, lda, ta, b, ldb, tb, M, N, K, C, N, epilogue=epi)
+    ref[ref.abs() > 3.4028235e38] *= float("inf")  # past the float32 range
+    assert torch.equal(C.isnan(), ref.isnan()) and torch.equal(C.isinf(), ref.isinf())
+    fin = ref.isfinite()
+    assert torch.equal(C[C.isinf()].sign().double(), ref[ref.isinf()].sign())
+    assert ((C.double() - ref).abs()[fin] <= bound(A, B, K)[fin]).all()
