@@ -188,6 +188,15 @@ typedef struct na_gemm_args {
 
 int na_gemm(const na_gemm_args* args, na_stream_t stream);
 
+/* The _slots forms of the calls whose workgroups each add to the same few addresses when
+ * they end (column sums, narrow weight gradients).  One address takes an atomic about every
+ * 0.18 us, so 512 workgroups that end together wait 90 us for each other.  Here
+ * they add to copy (workgroup mod slots) of each such destination, `slot_stride` floats after
+ * the previous one; the caller zeroes slots copies and sums them afterwards.  slots = 1 is
+ * the plain call. */
+int na_gemm_slots(const na_gemm_args* args, int32_t slots, int64_t slot_stride,
+                  na_stream_t stream); /* colsum */
+
 /* Tap increments of the BF16 4-tap numerical gradient
  * (projects/neuralangelo/utils/modules.py:157-175 with the SDF MLP of
  * projects/neuralangelo/utils/mlp.py:55-69), on the weights-stationary kernel.
@@ -230,6 +239,13 @@ int na_taps_increment_bwd(const void* D, int64_t ld_d, int64_t M, int64_t K, con
                           int64_t ld_dpre, void* centre, int64_t ld_centre, void* q,
                           int64_t ld_q, float* db0, float* dws, float* work,
                           int32_t work_holds_dz, na_stream_t stream);
+int na_taps_increment_bwd_slots(const void* D, int64_t ld_d, int64_t M, int64_t K, const void* W,
+                                int64_t ldw, int64_t N, const float* zc, int64_t ld_zc,
+                                const float* ws, float beta, const float* dds, void* dpre,
+                                int64_t ld_dpre, void* centre, int64_t ld_centre, void* q,
+                                int64_t ld_q, float* db0, float* dws, float* work,
+                                int32_t work_holds_dz, int32_t slots, int64_t slot_stride,
+                                na_stream_t stream); /* db0, dws */
 
 /* Maximum partial-product floats of na_gemm_wgrad_static (80 MiB per device):
  * every weight gradient of the train step fits (the largest, the 280-wide colour
@@ -281,6 +297,12 @@ int na_linear_narrow_bwd(const void* X, int64_t ldx, int32_t x_dtype, int64_t M,
                          void* dX, int64_t lddx, int32_t dx_dtype, int32_t add_dx,
                          const void* Y, int64_t ldy, int32_t y_dtype, int32_t dact,
                          float act_beta, float* dx_colsum, na_stream_t stream);
+int na_linear_narrow_bwd_slots(const void* X, int64_t ldx, int32_t x_dtype, int64_t M, int64_t K,
+                               const float* W, int32_t N, const float* dpre, float* dW, float* db,
+                               void* dX, int64_t lddx, int32_t dx_dtype, int32_t add_dx,
+                               const void* Y, int64_t ldy, int32_t y_dtype, int32_t dact,
+                               float act_beta, float* dx_colsum, int32_t slots,
+                               int64_t slot_stride, na_stream_t stream); /* dW, db, dx_colsum */
 
 /* out[m, n] = dy[m*ld_dy + n] * act'(y[m*ld_y + n]) for n < N (derivative through
  * the activation output y, as na_gemm's dact); colsum[n] += out[m,n] when
@@ -288,6 +310,10 @@ int na_linear_narrow_bwd(const void* X, int64_t ldx, int32_t x_dtype, int64_t M,
 int na_act_grad(const void* dy, int64_t ld_dy, int32_t dy_dtype, const void* y, int64_t ld_y,
                 int32_t y_dtype, int64_t M, int64_t N, int32_t act, float act_beta, void* out,
                 int64_t ld_out, int32_t out_dtype, float* colsum, na_stream_t stream);
+int na_act_grad_slots(const void* dy, int64_t ld_dy, int32_t dy_dtype, const void* y, int64_t ld_y,
+                      int32_t y_dtype, int64_t M, int64_t N, int32_t act, float act_beta,
+                      void* out, int64_t ld_out, int32_t out_dtype, float* colsum, int32_t slots,
+                      int64_t slot_stride, na_stream_t stream); /* colsum */
 
 /* Weight normalisation W = g * v / ||v||_row (v [N,K], g [N]); optionally also
  * writes a bf16 copy Wb.  Backward writes (does not accumulate)

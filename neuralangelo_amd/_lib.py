@@ -96,6 +96,7 @@ _SIGNATURES = {
     "na_hashgrid_fwd": (ctypes.c_int, [_PGRID, _P, _I64, _P, _I32, _P, _I32, _I32, _P]),
     "na_hashgrid_bwd": (ctypes.c_int, [_PGRID, _P, _I64, _P, _I32, _P, _I32, _P]),
     "na_gemm": (ctypes.c_int, [_PGEMM, _P]),
+    "na_gemm_slots": (ctypes.c_int, [_PGEMM, _I32, _I64, _P]),
     "na_gemm_wgrad_workspace": (ctypes.c_int64, [_PGEMM]),
     "na_gemm_wgrad_static": (ctypes.c_int, [_PGEMM, _P]),
     "na_taps_increment_fwd": (ctypes.c_int, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _P,
@@ -103,10 +104,15 @@ _SIGNATURES = {
     "na_taps_increment_bwd": (ctypes.c_int, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _P,
                                              _F32, _P, _P, _I64, _P, _I64, _P, _I64, _P, _P, _P,
                                              _I32, _P]),
+    "na_taps_increment_bwd_slots": (ctypes.c_int, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64,
+                                                   _P, _F32, _P, _P, _I64, _P, _I64, _P, _I64, _P,
+                                                   _P, _P, _I32, _I32, _I64, _P]),
     "na_colsum": (ctypes.c_int, [_P, _I64, _I32, _I64, _I64, _P, _P]),
     "na_head_sum": (ctypes.c_int, [_P, _I32, _I64, _P, _P, _P]),
     "na_linear_narrow_fwd": (ctypes.c_int, [_P, _I64, _I32, _I64, _I64, _P, _P, _I32, _I32, _P, _P]),
     "na_linear_narrow_bwd": (ctypes.c_int, [_P, _I64, _I32, _I64, _I64, _P, _I32, _P, _P, _P, _P, _I64, _I32, _I32, _P, _I64, _I32, _I32, _F32, _P, _P]),
+    "na_linear_narrow_bwd_slots": (ctypes.c_int, [_P, _I64, _I32, _I64, _I64, _P, _I32, _P, _P, _P, _P, _I64, _I32, _I32, _P, _I64, _I32, _I32, _F32, _P, _I32, _I64, _P]),
+    "na_act_grad_slots": (ctypes.c_int, [_P, _I64, _I32, _P, _I64, _I32, _I64, _I64, _I32, _F32, _P, _I64, _I32, _P, _I32, _I64, _P]),
     "na_act_grad": (ctypes.c_int, [_P, _I64, _I32, _P, _I64, _I32, _I64, _I64, _I32, _F32, _P, _I64, _I32, _P, _P]),
     "na_weight_norm_fwd": (ctypes.c_int, [_P, _P, _I64, _I64, _P, _P, _I32, _I64, _P]),
     "na_weight_norm_bwd": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _P, _P]),

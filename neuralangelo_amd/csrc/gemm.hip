@@ -54,6 +54,9 @@ struct EpiParams {
   void* tap_q;
   int64_t tap_ld_q;
   float* colsum2;
+  // column sums go to copy blockIdx.x % slots of the destination (slot_offset)
+  int slots;
+  int64_t slot_stride;
 };
 
 struct GemmParams {
@@ -65,6 +68,14 @@ struct GemmParams {
   int64_t k_chunk;
   EpiParams e;
 };
+
+// Sums that every workgroup adds to the same few addresses when it ends: one address takes
+// an atomic about every 0.18 us, so 512 workgroups that end together wait 90 us for
+// each other.  The caller can pass several zeroed copies of the destination,
+// `stride` floats apart, and sum them afterwards; workgroups take them in turn.
+__device__ inline int64_t slot_offset(int slots, int64_t stride) {
+  return slots > 1 ? (int64_t)(blockIdx.x % (uint32_t)slots) * stride : 0;
+}
 
 __device__ inline float act_forward(int act, float v, float beta) {
   if (act == NA_ACT_RELU) return v > 0.0f ? v : 0.0f;
@@ -355,7 +366,7 @@ __device__ __attribute__((always_inline)) inline void gemm_epilogue(
     }
     __syncthreads();
   }
-  if (e.colsum && ncol) atomic_add_f32(e.colsum + n, csum);
+  if (e.colsum && ncol) atomic_add_f32(e.colsum + slot_offset(e.slots, e.slot_stride) + n, csum);
 }
 
 // Two LDS stages: the next K-tile is fetched into registers while the MFMAs
@@ -632,7 +643,8 @@ narrow_bwd_vec_kernel(const TX* __restrict__ X, int64_t ldx, int64_t M, int64_t 
                       const float* __restrict__ W, int N, const float* __restrict__ dpre,
                       float* __restrict__ dW, float* __restrict__ db, TDX* __restrict__ dX,
                       int64_t lddx, int add_dx, const void* Y, int64_t ldy, int y_dtype,
-                      int dact, float beta, float* __restrict__ dx_colsum) {
+                      int dact, float beta, float* __restrict__ dx_colsum, int slots,
+                      int64_t slot_stride) {
   const int lane = threadIdx.x & 63;
   const int hl = lane & 31, half = lane >> 5;
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -821,13 +833,14 @@ narrow_bwd_vec_kernel(const TX* __restrict__ X, int64_t ldx, int64_t M, int64_t 
 #pragma unroll
       for (int n = 0; n < NM; ++n) gb[n] += r[(NM + 1) * KC * 256 + n];
     }
+    const int64_t so = slot_offset(slots, slot_stride);
     for (int n = 0; n < N; ++n) {
 #pragma unroll
       for (int c = 0; c < KC; ++c)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int64_t k = 8 * hl + 256 * c + e;
-          if (k < K) atomic_add_f32(dW + n * K + k, gw[n][c][e]);
+          if (k < K) atomic_add_f32(dW + so + n * K + k, gw[n][c][e]);
         }
     }
     if (dX && dx_colsum) {
@@ -836,11 +849,11 @@ narrow_bwd_vec_kernel(const TX* __restrict__ X, int64_t ldx, int64_t M, int64_t 
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int64_t k = 8 * hl + 256 * c + e;
-          if (k < K) atomic_add_f32(dx_colsum + k, cs[c][e]);
+          if (k < K) atomic_add_f32(dx_colsum + so + k, cs[c][e]);
         }
     }
     if (hl == 0)
-      for (int n = 0; n < N; ++n) atomic_add_f32(db + n, gb[n]);
+      for (int n = 0; n < N; ++n) atomic_add_f32(db + so + n, gb[n]);
   }
 }
 
@@ -849,7 +862,7 @@ template <typename TD, typename TY, typename TO>
 __global__ void __launch_bounds__(256)
 act_grad_kernel(const TD* __restrict__ dy, int64_t ld_dy, const TY* __restrict__ y, int64_t ld_y,
                 int64_t M, int64_t N, int act, float beta, TO* __restrict__ out, int64_t ld_out,
-                float* __restrict__ colsum) {
+                float* __restrict__ colsum, int slots, int64_t slot_stride) {
   // block: 256 threads = 64 columns x 4 row lanes; grid.x over row chunks, grid.y over columns
   const int64_t n = (int64_t)blockIdx.y * 64 + (threadIdx.x & 63);
   const int rl = threadIdx.x >> 6;
@@ -870,7 +883,7 @@ act_grad_kernel(const TD* __restrict__ dy, int64_t ld_dy, const TY* __restrict__
     __syncthreads();
     if (rl == 0 && n < N) {
       float s = red[threadIdx.x] + red[threadIdx.x + 64] + red[threadIdx.x + 128] + red[threadIdx.x + 192];
-      atomic_add_f32(colsum + n, s);
+      atomic_add_f32(colsum + slot_offset(slots, slot_stride) + n, s);
     }
   }
 }
@@ -1757,7 +1770,7 @@ gemm_bf16_nn_persist_kernel(GemmParams p) {
       if (p.e.colsum) {
         const uint32_t nxt = tile + gridDim.x;
         if (jt + 1 == my_tiles || nxt / n_mt != tile / n_mt)
-          persist_flush_colsum<WN>(p.e.colsum, p.N, n0 + wn * 64, lane, csum,
+          persist_flush_colsum<WN>(p.e.colsum + slot_offset(p.e.slots, p.e.slot_stride), p.N, n0 + wn * 64, lane, csum,
                                    reinterpret_cast<float*>(smem + NS * PT::STAGE_EL * 2), wm, wn);
       }
     }
@@ -2102,7 +2115,7 @@ gemm_f32_kernel(GemmParams p, int64_t parts) {
     if (e.colsum) {
       __syncthreads();
       for (int c = tid; c < BN; c += GNT)
-        if (n0 + c < p.N) atomic_add_f32(e.colsum + n0 + c, s_col[c]);
+        if (n0 + c < p.N) atomic_add_f32(e.colsum + slot_offset(e.slots, e.slot_stride) + n0 + c, s_col[c]);
     }
   } else {
     static_assert(MODE != F3_GENERAL || NB == 4, "the staged epilogue takes 64 columns at a time");
@@ -2575,12 +2588,13 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
     }
   }
   if constexpr (KIND == PK_DACT) {
-    if (e.colsum) ws_flush_colsum(e.colsum + nw + 8 * h, cs, lane);
+    if (e.colsum)
+      ws_flush_colsum(e.colsum + slot_offset(e.slots, e.slot_stride) + nw + 8 * h, cs, lane);
   }
   if constexpr (kTB) {
     // lane j adds entry j of the wave's sums: (sum j / 32, h, group, column)
     const int j = lane & 31, hh = j >> 4, gq = (j >> 3) & 1, c = j & 7;
-    float* dst = lane < 32 ? e.colsum : e.colsum2;
+    float* dst = (lane < 32 ? e.colsum : e.colsum2) + slot_offset(e.slots, e.slot_stride);
     atomic_add_f32(dst + nw + 16 * gq + 8 * hh + c, tb_sums[wave * 64 + lane]);
   }
   __builtin_amdgcn_s_waitcnt(0xF70);  // no buffer-to-LDS load outlives the workgroup
@@ -2610,7 +2624,7 @@ taps_increment_bwd_kernel(const float* __restrict__ dz, int64_t P, int N,
                           const float* __restrict__ dds, bf16_t* __restrict__ dpre,
                           int64_t ld_dpre, bf16_t* __restrict__ centre, int64_t ld_centre,
                           bf16_t* __restrict__ q, int64_t ld_q, float* __restrict__ db0,
-                          float* __restrict__ dws) {
+                          float* __restrict__ dws, int slots, int64_t slot_stride) {
   __shared__ float red[2][kTibBlock][4];
   const int cpp = N / 4;               // 4-column chunks per point (64 or 32)
   const int ppb = kTibBlock / cpp;     // points per workgroup pass (4 or 8)
@@ -2666,10 +2680,11 @@ taps_increment_bwd_kernel(const float* __restrict__ dz, int64_t P, int N,
         hs[c] += red[1][k * cpp + chunk][c];
       }
     }
+    const int64_t so = slot_offset(slots, slot_stride);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      atomic_add_f32(db0 + c0 + c, cs[c]);
-      atomic_add_f32(dws + c0 + c, hs[c]);
+      atomic_add_f32(db0 + so + c0 + c, cs[c]);
+      atomic_add_f32(dws + so + c0 + c, hs[c]);
     }
   }
 }
@@ -3160,7 +3175,8 @@ template <typename TD, typename TY, typename TO>
 __global__ void __launch_bounds__(256)
 act_grad_vec_kernel(const TD* __restrict__ dy, int64_t ld_dy, const TY* __restrict__ y, int64_t ld_y,
                     int64_t M, int64_t N, int act, float beta, TO* __restrict__ out, int64_t ld_out,
-                    float* __restrict__ colsum, int64_t rows_per_block) {
+                    float* __restrict__ colsum, int slots, int64_t slot_stride,
+                    int64_t rows_per_block) {
   __shared__ float red[256 * 8];
   const int cpr = (int)(N / 8);
   const int c = threadIdx.x % cpr, r = threadIdx.x / cpr, lanes = 256 / cpr;
@@ -3207,7 +3223,7 @@ act_grad_vec_kernel(const TD* __restrict__ dy, int64_t ld_dy, const TY* __restri
       for (int k = 0; k < 8; ++k) {
         float s = 0.0f;
         for (int q = 0; q < lanes; ++q) s += red[k * 256 + q * cpr + c];
-        atomic_add_f32(colsum + 8 * c + k, s);
+        atomic_add_f32(colsum + slot_offset(slots, slot_stride) + 8 * c + k, s);
       }
     }
   }
@@ -3226,7 +3242,7 @@ static int taps_increment(bool backward, const void* D, int64_t ld_d, int64_t M,
                           const float* ws, float beta, float* head_out, const float* dds,
                           void* dpre, int64_t ld_dpre, void* centre, int64_t ld_centre,
                           void* q, int64_t ld_q, float* db0, float* dws, float* work,
-                          int work_holds_dz, hipStream_t s) {
+                          int work_holds_dz, int slots, int64_t slot_stride, hipStream_t s) {
   NA_CHECK_ARG(M >= 0 && M % GBM == 0, "rows must be a multiple of 128 (pad the points to 32)");
   NA_CHECK_ARG(N == 256 || N == 128, "layer width must be 128 or 256");
   const int64_t nk = ceil_div(K, (int64_t)kNNBK);
@@ -3280,6 +3296,7 @@ static int taps_increment(bool backward, const void* D, int64_t ld_d, int64_t M,
     p.e.tap_centre = centre; p.e.tap_ld_centre = ld_centre;
     p.e.tap_q = q; p.e.tap_ld_q = ld_q;
     p.e.colsum = db0; p.e.colsum2 = dws;
+    p.e.slots = slots; p.e.slot_stride = slot_stride;
     if (nwv == 8) launch_ws<8>((int)nk, PK_TAPS_BWD, wg, p, s);
     else launch_ws<4>((int)nk, PK_TAPS_BWD, wg, p, s);
     NA_CHECK_LAUNCH();
@@ -3304,7 +3321,7 @@ static int taps_increment(bool backward, const void* D, int64_t ld_d, int64_t M,
       std::max<int64_t>(1, std::min<int64_t>(groups, (int64_t)ncu * tune_value(TUNE_TIB_WG_PER_CU)));
   hipLaunchKernelGGL(taps_increment_bwd_kernel, dim3((unsigned)grid), dim3(kTibBlock), 0, s,
                      (const float*)work, P, (int)N, zc, ld_zc, ws, beta, dds, (bf16_t*)dpre,
-                     ld_dpre, (bf16_t*)centre, ld_centre, (bf16_t*)q, ld_q, db0, dws);
+                     ld_dpre, (bf16_t*)centre, ld_centre, (bf16_t*)q, ld_q, db0, dws, slots, slot_stride);
   NA_CHECK_LAUNCH();
   return NA_OK;
 }
@@ -3359,7 +3376,7 @@ extern "C" int na_taps_increment_fwd(const void* D, int64_t ld_d, int64_t M, int
                                      float* dz_out, na_stream_t stream) {
   return taps_increment(false, D, ld_d, M, K, W, ldw, N, zc, ld_zc, ws, beta, head_out,
                         nullptr, nullptr, 0, nullptr, 0, nullptr, 0, nullptr, nullptr, dz_out, 0,
-                        (hipStream_t)stream);
+                        1, 0, (hipStream_t)stream);
 }
 
 extern "C" int na_taps_increment_bwd(const void* D, int64_t ld_d, int64_t M, int64_t K,
@@ -3368,9 +3385,23 @@ extern "C" int na_taps_increment_bwd(const void* D, int64_t ld_d, int64_t M, int
                                      void* dpre, int64_t ld_dpre, void* centre, int64_t ld_centre,
                                      void* q, int64_t ld_q, float* db0, float* dws, float* work,
                                      int32_t work_holds_dz, na_stream_t stream) {
+  return na_taps_increment_bwd_slots(D, ld_d, M, K, W, ldw, N, zc, ld_zc, ws, beta, dds, dpre,
+                                     ld_dpre, centre, ld_centre, q, ld_q, db0, dws, work,
+                                     work_holds_dz, 1, 0, stream);
+}
+
+extern "C" int na_taps_increment_bwd_slots(const void* D, int64_t ld_d, int64_t M, int64_t K,
+                                           const void* W, int64_t ldw, int64_t N, const float* zc,
+                                           int64_t ld_zc, const float* ws, float beta,
+                                           const float* dds, void* dpre, int64_t ld_dpre,
+                                           void* centre, int64_t ld_centre, void* q, int64_t ld_q,
+                                           float* db0, float* dws, float* work,
+                                           int32_t work_holds_dz, int32_t slots,
+                                           int64_t slot_stride, na_stream_t stream) {
+  NA_CHECK_ARG(slots >= 1 && slot_stride >= 0, "bad slots");
   return taps_increment(true, D, ld_d, M, K, W, ldw, N, zc, ld_zc, ws, beta, nullptr, dds,
                         dpre, ld_dpre, centre, ld_centre, q, ld_q, db0, dws, work,
-                        work_holds_dz, (hipStream_t)stream);
+                        work_holds_dz, slots, slot_stride, (hipStream_t)stream);
 }
 
 extern "C" int64_t na_gemm_wgrad_workspace(const na_gemm_args* a) {
@@ -3381,7 +3412,13 @@ extern "C" int64_t na_gemm_wgrad_workspace(const na_gemm_args* a) {
 }
 
 extern "C" int na_gemm(const na_gemm_args* a, na_stream_t stream) {
+  return na_gemm_slots(a, 1, 0, stream);
+}
+
+extern "C" int na_gemm_slots(const na_gemm_args* a, int32_t slots, int64_t slot_stride,
+                             na_stream_t stream) {
   NA_CHECK_ARG(a != nullptr, "args is null");
+  NA_CHECK_ARG(slots >= 1 && slot_stride >= 0, "bad slots");
   NA_CHECK_ARG(a->M >= 0 && a->N >= 0 && a->K >= 0, "negative size");
   if (a->M == 0 || a->N == 0) return NA_OK;
   NA_CHECK_ARG(a->in_dtype == NA_F32 || a->in_dtype == NA_BF16, "in_dtype must be F32 or BF16");
@@ -3419,6 +3456,7 @@ extern "C" int na_gemm(const na_gemm_args* a, na_stream_t stream) {
   p.e.bias = a->bias; p.e.act = a->act; p.e.beta = a->act_beta;
   p.e.dact_y = a->dact_y; p.e.ld_dact = a->ld_dact; p.e.dact_dtype = a->dact_dtype; p.e.dact = a->dact;
   p.e.r1_a = a->r1_a; p.e.r1_b = a->r1_b; p.e.colsum = a->colsum;
+  p.e.slots = slots; p.e.slot_stride = slot_stride;
   p.e.z_out = a->z_out; p.e.ld_z = a->ld_z; p.e.zc = a->zc; p.e.ld_zc = a->ld_zc;
   p.e.zc_rows = a->zc_rows; p.e.head_w = a->head_w; p.e.head_out = a->head_out;
   dim3 grid((unsigned)ceil_div(a->M, GBM), (unsigned)ceil_div(a->N, GBN), (unsigned)nsplit);
@@ -3488,6 +3526,18 @@ extern "C" int na_linear_narrow_bwd(const void* X, int64_t ldx, int32_t x_dtype,
                                     int32_t add_dx, const void* Y, int64_t ldy, int32_t y_dtype,
                                     int32_t dact, float act_beta, float* dx_colsum,
                                     na_stream_t stream) {
+  return na_linear_narrow_bwd_slots(X, ldx, x_dtype, M, K, W, N, dpre, dW, db, dX, lddx, dx_dtype,
+                                    add_dx, Y, ldy, y_dtype, dact, act_beta, dx_colsum, 1, 0, stream);
+}
+
+extern "C" int na_linear_narrow_bwd_slots(const void* X, int64_t ldx, int32_t x_dtype, int64_t M,
+                                          int64_t K, const float* W, int32_t N, const float* dpre,
+                                          float* dW, float* db, void* dX, int64_t lddx,
+                                          int32_t dx_dtype, int32_t add_dx, const void* Y,
+                                          int64_t ldy, int32_t y_dtype, int32_t dact,
+                                          float act_beta, float* dx_colsum, int32_t slots,
+                                          int64_t slot_stride, na_stream_t stream) {
+  NA_CHECK_ARG(slots >= 1 && slot_stride >= 0, "bad slots");
   NA_CHECK_ARG(N >= 1 && N <= kNarrowMax, "N must be in [1, 4]");
   NA_CHECK_ARG(M >= 0 && K >= 1, "bad sizes");
   if (M == 0) return NA_OK;
@@ -3508,7 +3558,7 @@ extern "C" int na_linear_narrow_bwd(const void* X, int64_t ldx, int32_t x_dtype,
 #define NA_NBWD_L(TX, TDX, KC, NM, XO)                                                         \
   hipLaunchKernelGGL((narrow_bwd_vec_kernel<TX, TDX, KC, NM, XO>), grid8, dim3(512), 0, s,     \
                      (const TX*)X, ldx, M, K, W, N, dpre, dW, db, (TDX*)dX, lddx, add_dx, Y,   \
-                     ldy, y_dtype, dact, act_beta, dx_colsum)
+                     ldy, y_dtype, dact, act_beta, dx_colsum, slots, slot_stride)
 #define NA_NBWD(TX, TDX, KC)                                                                   \
   do {                                                                                         \
     if (N == 1) {                                                                              \
@@ -3540,6 +3590,16 @@ extern "C" int na_act_grad(const void* dy, int64_t ld_dy, int32_t dy_dtype, cons
                            int64_t ld_y, int32_t y_dtype, int64_t M, int64_t N, int32_t act,
                            float act_beta, void* out, int64_t ld_out, int32_t out_dtype,
                            float* colsum, na_stream_t stream) {
+  return na_act_grad_slots(dy, ld_dy, dy_dtype, y, ld_y, y_dtype, M, N, act, act_beta, out, ld_out,
+                           out_dtype, colsum, 1, 0, stream);
+}
+
+extern "C" int na_act_grad_slots(const void* dy, int64_t ld_dy, int32_t dy_dtype, const void* y,
+                                 int64_t ld_y, int32_t y_dtype, int64_t M, int64_t N, int32_t act,
+                                 float act_beta, void* out, int64_t ld_out, int32_t out_dtype,
+                                 float* colsum, int32_t slots, int64_t slot_stride,
+                                 na_stream_t stream) {
+  NA_CHECK_ARG(slots >= 1 && slot_stride >= 0, "bad slots");
   NA_CHECK_ARG(M >= 0 && N >= 0, "bad sizes");
   if (M == 0 || N == 0) return NA_OK;
   NA_CHECK_ARG(dy && y && out, "null pointer");
@@ -3549,31 +3609,33 @@ extern "C" int na_act_grad(const void* dy, int64_t ld_dy, int32_t dy_dtype, cons
   const bool vec = N % 8 == 0 && 256 % (N / 8) == 0 && ld_dy % 8 == 0 && ld_y % 8 == 0 &&
                    ld_out % 8 == 0 && ((uintptr_t)dy | (uintptr_t)y | (uintptr_t)out) % 16 == 0 &&
                    (d16 || ld_dy % 4 == 0);
-  if (vec && d16 && y16) {
+  if (vec && d16 == y16 && (d16 || !o16)) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
       cus = 256;
+    // short row ranges for few rows: two batches of a thread's rows fill the CUs down
+    // to 4,096 rows (64 rows a block left three CUs in four idle there)
     const int64_t lanes = 256 / (N / 8);
     int64_t blocks = 2 * (int64_t)cus;
     int64_t rpb = ceil_div(ceil_div(M, blocks), lanes) * lanes;
-    if (rpb < 64) rpb = 64;
+    if (rpb < 2 * lanes) rpb = 2 * lanes;
     blocks = ceil_div(M, rpb);
-    if (o16)
-      hipLaunchKernelGGL((act_grad_vec_kernel<bf16_t, bf16_t, bf16_t>), dim3((unsigned)blocks), dim3(256), 0,
-                         s, (const bf16_t*)dy, ld_dy, (const bf16_t*)y, ld_y, M, N, act, act_beta,
-                         (bf16_t*)out, ld_out, colsum, rpb);
-    else
-      hipLaunchKernelGGL((act_grad_vec_kernel<bf16_t, bf16_t, float>), dim3((unsigned)blocks), dim3(256), 0,
-                         s, (const bf16_t*)dy, ld_dy, (const bf16_t*)y, ld_y, M, N, act, act_beta,
-                         (float*)out, ld_out, colsum, rpb);
+#define NA_ACTV(TD, TO)                                                                            \
+  hipLaunchKernelGGL((act_grad_vec_kernel<TD, TD, TO>), dim3((unsigned)blocks), dim3(256), 0, s,  \
+                     (const TD*)dy, ld_dy, (const TD*)y, ld_y, M, N, act, act_beta, (TO*)out,     \
+                     ld_out, colsum, slots, slot_stride, rpb)
+    if (!d16) NA_ACTV(float, float);
+    else if (o16) NA_ACTV(bf16_t, bf16_t);
+    else NA_ACTV(bf16_t, float);
+#undef NA_ACTV
     NA_CHECK_LAUNCH();
     return NA_OK;
   }
   dim3 grid((unsigned)ceil_div(M, 256), (unsigned)ceil_div(N, 64));
 #define NA_ACTG(TD, TY, TO)                                                                   \
   hipLaunchKernelGGL((act_grad_kernel<TD, TY, TO>), grid, dim3(256), 0, s, (const TD*)dy, ld_dy, \
-                     (const TY*)y, ld_y, M, N, act, act_beta, (TO*)out, ld_out, colsum)
+                     (const TY*)y, ld_y, M, N, act, act_beta, (TO*)out, ld_out, colsum, slots, slot_stride)
   if (!d16 && !y16 && !o16) NA_ACTG(float, float, float);
   else if (!d16 && !y16 && o16) NA_ACTG(float, float, bf16_t);
   else if (!d16 && y16 && !o16) NA_ACTG(float, bf16_t, float);

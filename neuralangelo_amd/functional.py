@@ -17,6 +17,7 @@ Compute dtype is float32 or bfloat16 (MFMA inputs); accumulation, the SDF
 head, weight gradients and every per-ray quantity are float32.
 """
 import ctypes
+import math
 
 import torch
 import torch.nn.functional as torch_F
@@ -73,10 +74,11 @@ def _s(t):
 def gemm(A, lda, trans_a, B, ldb, trans_b, M, N, K, C, ldc, epilogue=NA_EPI_STORE, bias=None,
          act=NA_ACT_NONE, beta=SOFTPLUS_BETA, dact=NA_ACT_NONE, dact_y=None, ld_dact=0,
          colsum=None, split_k=1, r1_a=None, r1_b=None, z_out=None, zc=None, zc_rows=0,
-         head_w=None, head_out=None, wgrad_partials=True):
+         head_w=None, head_out=None, wgrad_partials=True, slots=(1, 0)):
     """C[m,n] = epi(sum_k A(m,k) B(n,k)) via na_gemm (see include/neuralangelo_amd.h).
     When the weight-gradient path runs the call, wgrad_partials gives it a workspace
-    for per-split partial products (split-ordered sums instead of atomics)."""
+    for per-split partial products (split-ordered sums instead of atomics).
+    slots: (copies, stride) of colsum, as SlotSums lays them out."""
     if A.dtype != B.dtype:
         raise RuntimeError(f"gemm operands must share a dtype ({A.dtype} vs {B.dtype})")
     a = _lib.GemmArgs()
@@ -107,7 +109,7 @@ def gemm(A, lda, trans_a, B, ldb, trans_b, M, N, K, C, ldc, epilogue=NA_EPI_STOR
         if n > 0:
             ws = torch.empty(n, dtype=torch.float32, device=C.device)
             a.wg_partials, a.wg_partials_len = ws.data_ptr(), n
-    _lib.call("na_gemm", ctypes.byref(a), _s(A))
+    _lib.call("na_gemm_slots", ctypes.byref(a), slots[0], slots[1], _s(A))
 
 
 def _zero_block(dev, *shapes):
@@ -126,6 +128,31 @@ def _zero_block(dev, *shapes):
         out.append(buf[o:o + n].view(*s))
         o += (n + 63) // 64 * 64
     return out
+
+
+class SlotSums:
+    """Accumulators of sums over `rows` rows that every workgroup adds to when it ends,
+    in several copies (na_gemm_slots): one zero-filled buffer, views of the first copy in
+    `first`, and one sum over the copies at the end.  Few rows need one copy: their
+    workgroups are few."""
+
+    def __init__(self, dev, rows, *shapes):
+        self.shapes = shapes
+        self.sizes = [math.prod(s) for s in shapes]
+        width = sum((n + 63) // 64 * 64 for n in self.sizes)
+        self.slots = (32 if rows >= 2048 else 1, width)
+        self.buf = torch.zeros(self.slots[0], width, device=dev)
+        self.first = self._views(self.buf[0])
+
+    def _views(self, row):
+        out, o = [], 0
+        for s, n in zip(self.shapes, self.sizes):
+            out.append(row[o:o + n].view(s))
+            o += (n + 63) // 64 * 64
+        return out
+
+    def sums(self):
+        return self._views(self.buf.sum(0)) if self.slots[0] > 1 else self.first
 
 
 def head_parts(N):
@@ -161,14 +188,14 @@ def linear_weight_grad(dpre, X, ldx, K, dW):
          split_k=_split_for(M))
 
 
-def act_grad(dy, y, act, out_dtype, colsum=None, n_cols=None):
+def act_grad(dy, y, act, out_dtype, colsum=None, n_cols=None, slots=(1, 0)):
     """dy * act'(y) over the first n_cols columns (row strides taken from the tensors)."""
     M = dy.shape[0]
     N = dy.shape[1] if n_cols is None else n_cols
     out = torch.empty(M, N, dtype=out_dtype, device=dy.device)
-    _lib.call("na_act_grad", _lib.ptr(dy), dy.stride(0), _code(dy), _lib.ptr(y), y.stride(0),
+    _lib.call("na_act_grad_slots", _lib.ptr(dy), dy.stride(0), _code(dy), _lib.ptr(y), y.stride(0),
               _code(y), M, N, act, SOFTPLUS_BETA, _lib.ptr(out), N, _code(out),
-              _lib.ptr(colsum), _s(dy))
+              _lib.ptr(colsum), slots[0], slots[1], _s(dy))
     return out
 
 
@@ -333,14 +360,23 @@ def _sdf_mlp_forward(X0, w, with_feat):
 
 
 class _SDFGrads:
-    """Weight-gradient accumulators of the SDF MLP (kernel layout, fp32)."""
+    """Weight-gradient accumulators of the SDF MLP (kernel layout, fp32): the layers'
+    weights, and the vectors b0, ws, bs, b1 (sums over the rows, in slots)."""
 
-    def __init__(self, w, dev, with_feat):
+    def __init__(self, w, dev, with_feat, rows):
         hid = w.hidden
-        shapes = [(hid, w.k0p), (hid,), (1, hid), (1,)] + ([(hid, hid), (hid,)] if with_feat else [])
-        z = _zero_block(dev, *shapes)
-        self.dW0p, self.db0, self.dws, self.dbs = z[:4]
-        self.dW1, self.db1 = (z[4], z[5]) if with_feat else (None, None)
+        z = _zero_block(dev, (hid, w.k0p), *([(hid, hid)] if with_feat else []))
+        self.dW0p, self.dW1 = z[0], z[1] if with_feat else None
+        self.sums = SlotSums(dev, rows, (hid,), (1, hid), (1,), *([(hid,)] if with_feat else []))
+        self.slots = self.sums.slots
+        self.db0, self.dws, self.dbs = self.sums.first[:3]
+        self.db1 = self.sums.first[3] if with_feat else None
+
+    def finish(self):
+        """The vectors hold their sums over the slots from here on."""
+        v = self.sums.sums()
+        self.db0, self.dws, self.dbs = v[:3]
+        self.db1 = v[3] if len(v) > 3 else None
 
 
 def _sdf_mlp_backward(X0, H0, FB, w, dsdf, dfeat, acc, dpre0=None, wgrad=True):
@@ -355,21 +391,23 @@ def _sdf_mlp_backward(X0, H0, FB, w, dsdf, dfeat, acc, dpre0=None, wgrad=True):
     if dpre0 is None:
         dpre0 = torch.empty(P, hid, dtype=cdt, device=dev)
     if has_feat:
-        dpre1 = act_grad(dfeat, FB, NA_ACT_SOFTPLUS, cdt, colsum=acc.db1, n_cols=hid)
+        dpre1 = act_grad(dfeat, FB, NA_ACT_SOFTPLUS, cdt, colsum=acc.db1, n_cols=hid,
+                         slots=acc.slots)
         linear_weight_grad(dpre1, H0, hid, hid, acc.dW1)
         # dpre0 = (dpre1 . W1 + dsdf ws) * softplus'(H0), db0 = column sums: one GEMM epilogue
         gemm(dpre1, hid, 0, _t(w.W1), hid, 0, P, hid, hid, dpre0, hid, dact=NA_ACT_SOFTPLUS,
-             dact_y=H0, ld_dact=hid, r1_a=dsdf.view(-1), r1_b=w.ws.view(-1), colsum=acc.db0)
+             dact_y=H0, ld_dact=hid, r1_a=dsdf.view(-1), r1_b=w.ws.view(-1), colsum=acc.db0,
+             slots=acc.slots)
         # dws = dsdf^T H0, dbs = sum dsdf (no input gradient from this call)
-        _lib.call("na_linear_narrow_bwd", _lib.ptr(H0), hid, _code(H0), P, hid, _lib.ptr(w.ws), 1,
+        _lib.call("na_linear_narrow_bwd_slots", _lib.ptr(H0), hid, _code(H0), P, hid, _lib.ptr(w.ws), 1,
                   _lib.ptr(dsdf), _lib.ptr(acc.dws), _lib.ptr(acc.dbs), None, hid, _code(dpre0), 0,
-                  None, hid, _code(H0), NA_ACT_NONE, SOFTPLUS_BETA, None, _s(X0))
+                  None, hid, _code(H0), NA_ACT_NONE, SOFTPLUS_BETA, None, *acc.slots, _s(X0))
     else:
         # dpre0 = (dsdf ws) * softplus'(H0); dws, dbs; db0 = column sums of dpre0
-        _lib.call("na_linear_narrow_bwd", _lib.ptr(H0), hid, _code(H0), P, hid, _lib.ptr(w.ws), 1,
+        _lib.call("na_linear_narrow_bwd_slots", _lib.ptr(H0), hid, _code(H0), P, hid, _lib.ptr(w.ws), 1,
                   _lib.ptr(dsdf), _lib.ptr(acc.dws), _lib.ptr(acc.dbs), _lib.ptr(dpre0), hid,
                   _code(dpre0), 0, _lib.ptr(H0), hid, _code(H0), NA_ACT_SOFTPLUS,
-                  SOFTPLUS_BETA, _lib.ptr(acc.db0), _s(X0))
+                  SOFTPLUS_BETA, _lib.ptr(acc.db0), *acc.slots, _s(X0))
     if wgrad:
         linear_weight_grad(dpre0, X0, w.k0p, w.k0p, acc.dW0p)
     return dpre0
@@ -421,8 +459,9 @@ class SDFNetFunction(torch.autograd.Function):
         points, X0, H0, FB = ctx.saved_tensors
         w, enc = ctx.w, ctx.enc
         P, dev = X0.shape[0], X0.device
-        acc = _SDFGrads(w, dev, ctx.with_feat)
+        acc = _SDFGrads(w, dev, ctx.with_feat, P)
         dpre0 = _sdf_mlp_backward(X0, H0, FB if ctx.with_feat else None, w, dsdf, dfeat, acc)
+        acc.finish()
         dW0 = w.unpermute_dW0(acc.dW0p)
         dtable = dinp = None
         if enc is not None and ctx.needs_input_grad[1]:
@@ -564,7 +603,7 @@ class SDFCentreTapsDeltaFunction(torch.autograd.Function):
         w, enc, ld_d = ctx.w, ctx.enc, ctx.ld_d
         P, dev, hid = pts.shape[0], pts.device, w.hidden
         P32 = Zc.shape[0]
-        acc = _SDFGrads(w, dev, True)
+        acc = _SDFGrads(w, dev, True, P)
         # the centre's own pre-activation gradient and the taps' shared rows, in
         # P32-row buffers (the tap product covers whole 128-row tiles)
         dpre_c = torch.empty(P32, hid, dtype=w.cdt, device=dev)
@@ -584,12 +623,13 @@ class SDFCentreTapsDeltaFunction(torch.autograd.Function):
         ctx.dz = None
         if dz is None and not fused:
             dz, held = torch.empty(4 * P32, hid, dtype=torch.float32, device=dev), 0
-        _lib.call("na_taps_increment_bwd", _lib.ptr(D), ld_d, 4 * P32, ld_d, _lib.ptr(W0d), ld_d,
+        _lib.call("na_taps_increment_bwd_slots", _lib.ptr(D), ld_d, 4 * P32, ld_d, _lib.ptr(W0d), ld_d,
                   hid, _lib.ptr(Zc), hid, _lib.ptr(w.ws), float(SOFTPLUS_BETA), _lib.ptr(dds_pm),
                   _lib.ptr(dpre_t), hid, _lib.ptr(dpre_c), hid, _lib.ptr(q), hid,
                   _lib.ptr(acc.db0), _lib.ptr(acc.dws), _lib.ptr(dz) if dz is not None else None,
-                  held if dz is not None else 0, _s(pts))
+                  held if dz is not None else 0, *acc.slots, _s(pts))
         del dz
+        acc.finish()
         # first-layer weights: centre rows x X0c, tap rows x D (hi part and point
         # offset), shared rows x sum_t D_t
         linear_weight_grad(dpre_c[:P], X0c, w.k0p, w.k0p, acc.dW0p)
@@ -631,11 +671,12 @@ def _centre_taps_backward(ctx, pts, X0c, H0c, FB, X0t, H0t, dsdf, dfeat, ds_taps
     ws, bs, enc, cdt/n_enc, n_enc/eps)."""
     w, enc = ctx.w, ctx.enc
     P, dev = pts.shape[0], pts.device
-    acc = _SDFGrads(w, dev, True)
+    acc = _SDFGrads(w, dev, True, P)
     dpre_c = _sdf_mlp_backward(X0c, H0c, FB, w, dsdf, dfeat, acc)
     dpre_t = _sdf_mlp_backward(X0t, H0t, None, w,
                                ds_taps.reshape(4 * P, 1) if ds_taps is not None else None,
                                None, acc)
+    acc.finish()
     dtable = None
     if ctx.needs_input_grad[1]:
         dXc = _encoder_grad(dpre_c, w)
@@ -779,26 +820,28 @@ class RGBNetFunction(torch.autograd.Function):
             dpre3 = dpre3 * out * (1 - out)
         dpre3 = dpre3.contiguous()
         dWs = [None] * n_lin
-        # every weight/bias gradient of the colour MLP in one zeroed block
-        z = _zero_block(dev, *[(b.shape[0],) for b in w.b], (3, hid),
-                        *[(hid, hid) for _ in range(n_lin - 2)], (hid, RGB_LD))
-        dbs = z[:n_lin]
-        dWs[-1] = z[n_lin]
-        dW_mid, dW0p = z[n_lin + 1:-1], z[-1]
+        # the weight gradients of the colour MLP in one zeroed block; the biases' and the
+        # last layer's, sums over the rows, in slots
+        z = _zero_block(dev, *[(hid, hid) for _ in range(n_lin - 2)], (hid, RGB_LD))
+        dW_mid, dW0p = z[:-1], z[-1]
+        acc = SlotSums(dev, P, *[(b.shape[0],) for b in w.b], (3, hid))
+        dbs, dW_last = acc.first[:n_lin], acc.first[n_lin]
         # last hidden layer's pre-activation gradient, written in the compute dtype
         dpre = torch.empty(P, hid, dtype=cdt, device=dev)
-        _lib.call("na_linear_narrow_bwd", _lib.ptr(Hs[-1]), hid, _code(Hs[-1]), P, hid,
-                  _lib.ptr(w.W_last), 3, _lib.ptr(dpre3), _lib.ptr(dWs[-1]), _lib.ptr(dbs[-1]),
+        _lib.call("na_linear_narrow_bwd_slots", _lib.ptr(Hs[-1]), hid, _code(Hs[-1]), P, hid,
+                  _lib.ptr(w.W_last), 3, _lib.ptr(dpre3), _lib.ptr(dW_last), _lib.ptr(dbs[-1]),
                   _lib.ptr(dpre), hid, _code(dpre), 0, _lib.ptr(Hs[-1]), hid, _code(Hs[-1]),
-                  NA_ACT_RELU, SOFTPLUS_BETA, _lib.ptr(dbs[-2]), _s(FB))
+                  NA_ACT_RELU, SOFTPLUS_BETA, _lib.ptr(dbs[-2]), *acc.slots, _s(FB))
         for li in range(n_lin - 2, 0, -1):
             X = Hs[li - 1]
             dWs[li] = dW_mid[li - 1]
             linear_weight_grad(dpre, X, hid, hid, dWs[li])
             dprev = torch.empty(P, hid, dtype=cdt, device=dev)
             gemm(dpre, hid, 0, _t(w.W[li]), hid, 0, P, hid, hid, dprev, hid, dact=NA_ACT_RELU,
-                 dact_y=X, ld_dact=hid, colsum=dbs[li - 1])
+                 dact_y=X, ld_dact=hid, colsum=dbs[li - 1], slots=acc.slots)
             dpre = dprev
+        sums = acc.sums()
+        dbs, dWs[-1] = sums[:n_lin], sums[n_lin]
         linear_weight_grad(dpre, FB, RGB_LD, RGB_LD, dW0p)
         dWs[0] = w.unpermute_dW0(dW0p)
         # input gradient in the compute dtype: the feature columns go back to the SDF
@@ -1002,12 +1045,14 @@ class LinearAct(torch.autograd.Function):
             d8 = torch.zeros(P, N8, dtype=dY.dtype, device=dY.device)
             d8[:, :N] = dY
             dY = d8
-        db = torch.zeros(N8, device=X.device)
         if ctx.act == NA_ACT_NONE:
             dpre = dY.to(X.dtype).contiguous()
-            db += dY.float().sum(0)
+            db = dY.float().sum(0)
         else:
-            dpre = act_grad(dY.contiguous(), Y, ctx.act, X.dtype, colsum=db, n_cols=N8)
+            acc = SlotSums(X.device, P, (N8,))
+            dpre = act_grad(dY.contiguous(), Y, ctx.act, X.dtype, colsum=acc.first[0], n_cols=N8,
+                            slots=acc.slots)
+            db = acc.sums()[0]
         dW = torch.zeros(N8, K, device=X.device)
         linear_weight_grad(dpre, X, K, K, dW)
         dX = None
