@@ -2147,25 +2147,29 @@ template <int NWV> struct WsCfg {
   static constexpr int ROWS = GBM / NWV;  // stage rows loaded per wave
 };
 
-// vmcnt(n) for n = 0 .. 15 (larger counts wait for 15, which is also safe)
+// vmcnt(n) for n = 0 .. 15 (larger counts wait for 15, which is also safe), and every
+// LDS read done: the barrier that follows frees the previous stage's slot, and a
+// wave's last reads of it may still be queued (the products that use them can come after
+// the barrier).  A stage past the last tile reads no memory and writes its zeros at
+// once, soon enough to overtake such a read.
 __device__ inline void ws_wait(int ahead) {
   switch (ahead) {
-    case 0: __builtin_amdgcn_s_waitcnt(0xF70); break;
-    case 1: __builtin_amdgcn_s_waitcnt(0xF71); break;
-    case 2: __builtin_amdgcn_s_waitcnt(0xF72); break;
-    case 3: __builtin_amdgcn_s_waitcnt(0xF73); break;
-    case 4: __builtin_amdgcn_s_waitcnt(0xF74); break;
-    case 5: __builtin_amdgcn_s_waitcnt(0xF75); break;
-    case 6: __builtin_amdgcn_s_waitcnt(0xF76); break;
-    case 7: __builtin_amdgcn_s_waitcnt(0xF77); break;
-    case 8: __builtin_amdgcn_s_waitcnt(0xF78); break;
-    case 9: __builtin_amdgcn_s_waitcnt(0xF79); break;
-    case 10: __builtin_amdgcn_s_waitcnt(0xF7A); break;
-    case 11: __builtin_amdgcn_s_waitcnt(0xF7B); break;
-    case 12: __builtin_amdgcn_s_waitcnt(0xF7C); break;
-    case 13: __builtin_amdgcn_s_waitcnt(0xF7D); break;
-    case 14: __builtin_amdgcn_s_waitcnt(0xF7E); break;
-    default: __builtin_amdgcn_s_waitcnt(0xF7F); break;
+    case 0: __builtin_amdgcn_s_waitcnt(0x070); break;
+    case 1: __builtin_amdgcn_s_waitcnt(0x071); break;
+    case 2: __builtin_amdgcn_s_waitcnt(0x072); break;
+    case 3: __builtin_amdgcn_s_waitcnt(0x073); break;
+    case 4: __builtin_amdgcn_s_waitcnt(0x074); break;
+    case 5: __builtin_amdgcn_s_waitcnt(0x075); break;
+    case 6: __builtin_amdgcn_s_waitcnt(0x076); break;
+    case 7: __builtin_amdgcn_s_waitcnt(0x077); break;
+    case 8: __builtin_amdgcn_s_waitcnt(0x078); break;
+    case 9: __builtin_amdgcn_s_waitcnt(0x079); break;
+    case 10: __builtin_amdgcn_s_waitcnt(0x07A); break;
+    case 11: __builtin_amdgcn_s_waitcnt(0x07B); break;
+    case 12: __builtin_amdgcn_s_waitcnt(0x07C); break;
+    case 13: __builtin_amdgcn_s_waitcnt(0x07D); break;
+    case 14: __builtin_amdgcn_s_waitcnt(0x07E); break;
+    default: __builtin_amdgcn_s_waitcnt(0x07F); break;
   }
 }
 

@@ -427,3 +427,17 @@ def test_increment_epilogue_large_steps_and_linear_region(cuda):
     assert torch.isfinite(got).all() and torch.isfinite(ho).all()
     assert ((got - y1).abs() <= 1e-5 * y1.abs() + 1e-6).all()
     assert (ho.cpu().double().sum(0) - dsp.sum(1)).abs().max() < 1e-4
+
+
+def test_gemm_weights_stationary_stage_reuse(cuda):
+    """One tile per workgroup and a long epilogue after it (column sums): the loads past
+    the last tile must not overwrite a stage that another wave still reads."""
+    M, N, K = 128 * 513, 128, 256
+    bf = torch.bfloat16
+    A, B = _rand((M, K), 51, 0.1).to(bf).to(cuda), _rand((N, K), 52, 0.1).to(bf).to(cuda)
+    Y = torch.relu(_rand((M, N), 53)).to(bf).to(cuda)
+    ref = (A.double() @ B.double().t()) * (Y > 0)
+    for _ in range(8):
+        C, cs = torch.empty(M, N, device=cuda), torch.zeros(N, device=cuda)
+        Fn.gemm(A, K, 0, B, K, 0, M, N, K, C, N, dact=NA_ACT_RELU, dact_y=Y, ld_dact=N, colsum=cs)
+        assert (C.double() - ref).abs().max() < 1e-5
