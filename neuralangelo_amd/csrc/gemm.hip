@@ -2129,11 +2129,11 @@ gemm_f32_kernel(GemmParams p, int64_t parts) {
 
 // ---------------------------------------------------------------------------
 // Weights-stationary GEMM for the 256-wide MLP layers: C = epi(A . B^T) with
-// N = 256, M a multiple of 128 and NK 32-wide K stages.  Eight waves each own
+// N = 256 and NK 32-wide K stages.  Eight waves each own
 // 32 output columns and hold those columns' weights over the whole K range in
 // registers (2 NK fragments of 8 bf16 per lane), so only activation rows
 // stream: 128 x 32 bf16 stages (8 KB, one buffer-to-LDS load per wave) in
-// kWsNS LDS slots, up to kWsNS - 1 of them in flight, and no weight tile is
+// kWsNS LDS slots, up to kWsNS - 2 of them in flight, and no weight tile is
 // re-read per row tile.  The products take the weights as the first MFMA
 // operand, which leaves one output row per lane (four 4-column groups); a
 // permlane32 swap between the two halves of the wave turns them into two
@@ -2146,32 +2146,6 @@ template <int NWV> struct WsCfg {
   static constexpr int NS = NWV == 8 ? 15 : 9;
   static constexpr int ROWS = GBM / NWV;  // stage rows loaded per wave
 };
-
-// vmcnt(n) for n = 0 .. 15 (larger counts wait for 15, which is also safe), and every
-// LDS read done: the barrier that follows frees the previous stage's slot, and a
-// wave's last reads of it may still be queued (the products that use them can come after
-// the barrier).  A stage past the last tile reads no memory and writes its zeros at
-// once, soon enough to overtake such a read.
-__device__ inline void ws_wait(int ahead) {
-  switch (ahead) {
-    case 0: __builtin_amdgcn_s_waitcnt(0x070); break;
-    case 1: __builtin_amdgcn_s_waitcnt(0x071); break;
-    case 2: __builtin_amdgcn_s_waitcnt(0x072); break;
-    case 3: __builtin_amdgcn_s_waitcnt(0x073); break;
-    case 4: __builtin_amdgcn_s_waitcnt(0x074); break;
-    case 5: __builtin_amdgcn_s_waitcnt(0x075); break;
-    case 6: __builtin_amdgcn_s_waitcnt(0x076); break;
-    case 7: __builtin_amdgcn_s_waitcnt(0x077); break;
-    case 8: __builtin_amdgcn_s_waitcnt(0x078); break;
-    case 9: __builtin_amdgcn_s_waitcnt(0x079); break;
-    case 10: __builtin_amdgcn_s_waitcnt(0x07A); break;
-    case 11: __builtin_amdgcn_s_waitcnt(0x07B); break;
-    case 12: __builtin_amdgcn_s_waitcnt(0x07C); break;
-    case 13: __builtin_amdgcn_s_waitcnt(0x07D); break;
-    case 14: __builtin_amdgcn_s_waitcnt(0x07E); break;
-    default: __builtin_amdgcn_s_waitcnt(0x07F); break;
-  }
-}
 
 __device__ inline void ws_issue(__amdgpu_buffer_rsrc_t r, uint32_t off, bf16_t* dst) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)dst, 16, off, 0, 0, 0);
@@ -2252,15 +2226,23 @@ template <int NWV, int NK, int KIND>
 __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kernel(GemmParams p) {
   constexpr int kWsNS = WsCfg<NWV>::NS;
   constexpr int LOADS = WsCfg<NWV>::ROWS / 16;
+  // The wait for a stage (vmcnt): memory operations complete in order, so all but the
+  // loads of the kWsNS - 3 stages issued after it and the operand loads of the tile's
+  // epilogue, where the stage was issued before them (in an earlier tile).  (Counting the stages alone
+  // made each tile's first stage wait for those operands: the tap product
+  // 1.62 ms at 3.16 M rows, 1.28 ms now.)
+  constexpr int kOperands = KIND == PK_DACT ? 8 : (KIND == PK_DELTA || KIND == PK_TAPS_FWD ? 16 : 0);
+  constexpr auto wait_code = [](int n) { return 0xF70 | (n & 15) | ((n >> 4) << 14); };
+  constexpr int kAhead = (kWsNS - 3) * LOADS;
+  static_assert(kAhead + kOperands < 64, "stage waits");
   __shared__ __attribute__((aligned(16))) unsigned char smem[kWsNS * kWsStage * 2];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 5;
   bf16_t* st0 = reinterpret_cast<bf16_t*>(smem);
   const bf16_t* A = (const bf16_t*)p.A;
   const EpiParams& e = p.e;
-  const uint32_t n_mt = (uint32_t)(p.M / GBM);
+  const uint32_t n_mt = (uint32_t)((p.M + GBM - 1) / GBM);
   const int64_t my_tiles = blockIdx.x < n_mt ? (n_mt - 1 - blockIdx.x) / gridDim.x + 1 : 0;
-  const int64_t total = my_tiles * NK;
   const int nw = wave * 32;  // first column of this wave
 
   // weights of row nw + lane % 32 of B: 8 k-values (offset 8 h) of each 16-wide step
@@ -2296,7 +2278,6 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
   const uint32_t avoff = (uint32_t)(arow * p.lda * 2 + achunk * 16);
   const uint32_t ablk = (uint32_t)(16 * p.lda * 2);  // byte step between a wave's blocks
   const int akofs = achunk * 8;
-  int64_t issued = 0;
   uint32_t is_tile = blockIdx.x;
   int is_t = 0, is_slot = 0;
   const char* is_a = reinterpret_cast<const char*>(A + (int64_t)is_tile * GBM * p.lda);
@@ -2309,7 +2290,6 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
     for (int u = 0; u < LOADS; ++u)
       ws_issue(rs, in_k ? avoff + u * ablk : kOobOffset,
                st0 + is_slot * kWsStage + (wave * LOADS + u) * 16 * kNNBK);
-    ++issued;
     is_slot = is_slot + 1 == kWsNS ? 0 : is_slot + 1;
     if (++is_t == NK) {
       is_t = 0;
@@ -2323,9 +2303,13 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
   // workgroup waits for them before it ends.  With a fixed count of loads per
   // iteration the compiler's waits for the per-tile operand registers below
   // count exactly the stage loads issued after them.
-  (void)total;
+// One slot stays free: at a stage's barrier a wave's last reads of the previous stage may
+  // still be queued (the products that use them can come after the barrier), so the
+  // load issued there goes to the slot of the stage before that.  (A stage past the last
+  // tile reads no memory and writes its zeros at once, soon enough to overtake such
+  // reads; waiting for them at the barrier instead cost the tap product 7 %.)
 #pragma unroll
-  for (int s = 0; s < kWsNS - 1; ++s) issue_next();
+  for (int s = 0; s < kWsNS - 2; ++s) issue_next();
 
   const float ib = 1.0f / e.beta;
   // derivative kind: rank-1 coefficients of the lane's columns and column sums
@@ -2360,9 +2344,11 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
   __shared__ float tb_sums[kTB ? NWV * 64 : 1];
   if constexpr (kTB) tb_sums[wave * 64 + lane] = 0.0f;
   int slot = 0;
-  int64_t g = 0;
   for (int64_t jt = 0; jt < my_tiles; ++jt) {
     const int64_t m0 = (int64_t)(blockIdx.x + (uint32_t)jt * gridDim.x) * GBM;
+    // rows past M (the last tile's): the stages hold zeros, operand loads repeat the last
+    // row, nothing is stored (the tap kinds have whole tiles)
+    const int last = p.M - 1 - m0 < GBM ? (int)(p.M - 1 - m0) : GBM - 1;
     // derivative kind: the tile's stored activations (bf16) and rank-1 row terms,
     // requested before this tile's stage loads
     uint4 yv[KIND == PK_DACT ? 4 : 1][2];
@@ -2401,7 +2387,8 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
     if constexpr (KIND == PK_DACT) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int64_t m = m0 + i * 32 + (lane & 31);
+        const int r = i * 32 + (lane & 31);
+        const int64_t m = m0 + (r < last ? r : last);
 #pragma unroll
         for (int gq = 0; gq < 2; ++gq)
           yv[i][gq] = *reinterpret_cast<const uint4*>((const bf16_t*)e.dact_y + m * e.ld_dact + nw + 16 * gq + 8 * h);
@@ -2414,9 +2401,10 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
 #pragma unroll
-    for (int t = 0; t < NK; ++t, ++g) {
-      ws_wait((int)(issued - g - 1) * LOADS);
-      __builtin_amdgcn_s_barrier();  // stage g landed in every wave; stage g-1 consumed
+    for (int t = 0; t < NK; ++t) {
+      if (t < kWsNS - 2) __builtin_amdgcn_s_waitcnt(wait_code(kAhead + kOperands));
+      else __builtin_amdgcn_s_waitcnt(wait_code(kAhead));
+      __builtin_amdgcn_s_barrier();  // stage g landed in every wave; stage g-2 consumed
       issue_next();
       const bf16_t* sa = st0 + slot * kWsStage;
       slot = slot + 1 == kWsNS ? 0 : slot + 1;
@@ -2440,6 +2428,7 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t m = m0 + i * 32 + (lane & 31);
+      const bool in = i * 32 + (lane & 31) <= last;
       float o[2][8];
       float hsum = 0.0f;
 #pragma unroll
@@ -2538,14 +2527,21 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
             y[2 * c] = __uint_as_float(yw[c] << 16);
             y[2 * c + 1] = __uint_as_float(yw[c] & 0xffff0000u);
           }
+          const float r1 = in ? r1v[i] : 0.0f;
+          // the activation is chosen per chunk, not per element (a branch each)
+          if (e.dact == NA_ACT_RELU) {
 #pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            float x = fmaf(r1v[i], rb[gq][c], o[gq][c]);
-            x = e.dact == NA_ACT_RELU ? (y[c] > 0.0f ? x : 0.0f)
-                                      : x * act_deriv_from_y(NA_ACT_SOFTPLUS, y[c], e.beta);
-            cs[gq][c] += x;
-            o[gq][c] = x;
+            for (int c = 0; c < 8; ++c) {
+              const float x = fmaf(r1, rb[gq][c], o[gq][c]);
+              o[gq][c] = y[c] > 0.0f ? x : 0.0f;
+            }
+          } else {
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+              o[gq][c] = fmaf(r1, rb[gq][c], o[gq][c]) * act_deriv_from_y(NA_ACT_SOFTPLUS, y[c], e.beta);
           }
+#pragma unroll
+          for (int c = 0; c < 8; ++c) cs[gq][c] += o[gq][c];
         } else if constexpr (KIND == PK_DELTA || KIND == PK_TAPS_FWD) {
           if constexpr (KIND == PK_TAPS_FWD) {
             // the increments themselves, kept for the backward when asked for
@@ -2563,7 +2559,7 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
 #pragma unroll
           for (int c = 0; c < 8; ++c) o[gq][c] += bb[gq][c];
           if constexpr (KIND == PK_BIAS_SOFTPLUS) {
-            if (e.z_out) vstore8(e.z_out + m * e.ld_z + col, o[gq]);
+            if (e.z_out && in) vstore8(e.z_out + m * e.ld_z + col, o[gq]);
           }
 #pragma unroll
           for (int c = 0; c < 8; ++c) {
@@ -2577,7 +2573,7 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
           }
         }
         const int64_t col = nw + 16 * gq + 8 * h;
-        if constexpr (KIND != PK_TAPS_FWD) {
+        if (KIND != PK_TAPS_FWD && in) {
           if (e.c_dtype == NA_BF16) vstore8((bf16_t*)e.C + m * e.ldc + col, o[gq]);
           else vstore8((float*)e.C + m * e.ldc + col, o[gq]);
         }
@@ -2586,7 +2582,7 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
         // row m over the wave's 32 columns: this lane's 16 and its partner's 16
         if (e.head_w) {
           hsum += __shfl_xor(hsum, 32);
-          if (h == 0) e.head_out[(int64_t)wave * p.M + m] = hsum;
+          if (h == 0 && in) e.head_out[(int64_t)wave * p.M + m] = hsum;
         }
       }
     }
@@ -2972,16 +2968,17 @@ static void launch_persist(int kind, int grid, const GemmParams& p, hipStream_t 
   }
 }
 
-// Weights-stationary path: N = 256 or 128, whole 128-row tiles, K of 5, 8 or 9
-// stages; bf16 activations for the derivative kind, stored rows in whole tiles
-// for the increment kind.
+// Weights-stationary path: N = 256 or 128, K of 5, 8 or 9 stages; bf16
+// activations for the derivative kind, stored rows in whole tiles for the
+// increment kind.  Any row count: 789,252 rows of a packed batch (not whole 128-row
+// tiles) x 256 x 256 took 356 us (derivative) and 336 us (ReLU) on the persistent
+// kernel, 226 and 162 us here.
 static int ws_stages(const na_gemm_args* a, int kind) {
   if (kind == PK_DACT && (a->dact_dtype != NA_BF16 || a->ld_dact % 8 || !aligned16(a->dact_y))) return 0;
   if (kind == PK_DELTA && (a->zc_rows % GBM || a->ld_zc % 4)) return 0;
   if ((a->z_out || a->head_w) && kind != PK_BIAS_SOFTPLUS && kind != PK_DELTA) return 0;
   if (a->z_out && a->ld_z % 4) return 0;
-  if ((a->N != 256 && a->N != 128) || a->M % GBM != 0 || a->K % 8 != 0 || a->lda % 8 || a->ldb % 8)
-    return 0;
+  if ((a->N != 256 && a->N != 128) || a->K % 8 != 0 || a->lda % 8 || a->ldb % 8) return 0;
   if (!aligned16(a->A) || !aligned16(a->B)) return 0;
   const int64_t nk = ceil_div(a->K, (int64_t)kNNBK);
   if (kind == PK_DELTA && nk != 5) return 0;  // the increment layer's width (K <= 160)
@@ -3470,7 +3467,7 @@ extern "C" int na_gemm_slots(const na_gemm_args* a, int32_t slots, int64_t slot_
   if (kind >= 0) {
     const int nk = ws_stages(a, kind);
     const int nwv = a->N == 256 ? 8 : 4;
-    const int wg = nk ? ws_grid(a->M / GBM, nwv) : 0;
+    const int wg = nk ? ws_grid(ceil_div(a->M, (int64_t)GBM), nwv) : 0;
     if (wg > 0) {
       if (nwv == 8) launch_ws<8>(nk, kind, wg, p, s);
       else launch_ws<4>(nk, kind, wg, p, s);
