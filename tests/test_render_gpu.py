@@ -273,3 +273,30 @@ def test_sdf_losses_many_samples(cuda):
                             outside.to(cuda))
     assert abs(e.item() - e_ref.item()) < 1e-5 * abs(e_ref.item()) + 1e-6
     assert abs(cc.item() - c_ref.item()) < 1e-5 * abs(c_ref.item()) + 1e-6
+
+
+@pytest.mark.parametrize("R, N, Nf", [(1, 2, 1), (5, 64, 16), (130, 80, 16), (3, 255, 256), (7, 80, 257)])
+@pytest.mark.parametrize("rows", ["sorted", "ties", "unsorted", "nan"])
+def test_hierarchical_merge_order(cuda, R, N, Nf, rows):
+    """The merge of every row is the two-pointer walk over the coarse and the returned fine
+    distances (coarse first on ties), also for rows out of order; both kernels (a wave for
+    four rays up to 256 fine samples, a lane per ray beyond)."""
+    g = torch.Generator().manual_seed(R + N)
+    d = torch.rand(R, N, generator=g) * 2 + 2
+    if rows != "unsorted":
+        d = d.sort(dim=1).values
+    if rows == "ties":
+        d = (d * 8).round() / 8
+    s = (d - 3.0) * -0.7 + 0.05 * torch.randn(R, N, generator=g)
+    if rows == "nan":
+        d[0, N // 2] = float("nan")
+    merged, fine, pc, pf = [t.cpu() for t in nerf_util.hierarchical_round(d.to(cuda), s.to(cuda), 64.0, Nf)]
+    for r in range(R):
+        dr, fr, i, j = d[r].tolist(), fine[r].tolist(), 0, 0
+        for k in range(N + Nf):
+            if j >= Nf or (i < N and not fr[j] < dr[i]):
+                want, at, i = dr[i], int(pc[r, i]), i + 1
+            else:
+                want, at, j = fr[j], int(pf[r, j]), j + 1
+            got = float(merged[r, k])
+            assert at == k and (got == want or (got != got and want != want)), (r, k)
