@@ -315,6 +315,17 @@ int na_act_grad_slots(const void* dy, int64_t ld_dy, int32_t dy_dtype, const voi
                       void* out, int64_t ld_out, int32_t out_dtype, float* colsum, int32_t slots,
                       int64_t slot_stride, na_stream_t stream); /* colsum */
 
+/* SDF values without autograd state, out[i] = bs + sum_n ws[n] softplus(W0 [enc(x_i), x_i]
+ * + b)_n, in one kernel (sampling passes, lattices).  W [N, ldw] of `dtype` (the table's
+ * type as well) in the kernel layout of na_sdf_input_fwd's rows: float32 [enc | x], bf16
+ * [enc | W_hi | W_hi | W_lo].  na_sdf_value_supported: 1 where this kernel covers the grid,
+ * type and hidden width N (16 levels of 4 or 8 features, N of 128 or 256), else 0. */
+int na_sdf_value_supported(const na_grid_desc* desc, int32_t dtype, int64_t N);
+int na_sdf_value(const na_grid_desc* desc, const float* points, int64_t n, float vmin, float vmax,
+                 const void* table, int32_t dtype, int32_t active_levels, const void* W,
+                 int64_t ldw, int64_t N, const float* b, const float* ws, const float* bs,
+                 float beta, float* out, na_stream_t stream);
+
 /* Weight normalisation W = g * v / ||v||_row (v [N,K], g [N]); optionally also
  * writes a bf16 copy Wb.  Backward writes (does not accumulate)
  * dg = sum_k dW*v/||v|| and dv = g/||v|| * (dW - dg * v/||v||). */

@@ -114,6 +114,8 @@ _SIGNATURES = {
     "na_linear_narrow_bwd_slots": (ctypes.c_int, [_P, _I64, _I32, _I64, _I64, _P, _I32, _P, _P, _P, _P, _I64, _I32, _I32, _P, _I64, _I32, _I32, _F32, _P, _I32, _I64, _P]),
     "na_act_grad_slots": (ctypes.c_int, [_P, _I64, _I32, _P, _I64, _I32, _I64, _I64, _I32, _F32, _P, _I64, _I32, _P, _I32, _I64, _P]),
     "na_act_grad": (ctypes.c_int, [_P, _I64, _I32, _P, _I64, _I32, _I64, _I64, _I32, _F32, _P, _I64, _I32, _P, _P]),
+    "na_sdf_value_supported": (ctypes.c_int, [_PGRID, _I32, _I64]),
+    "na_sdf_value": (ctypes.c_int, [_PGRID, _P, _I64, _F32, _F32, _P, _I32, _I32, _P, _I64, _I64, _P, _P, _P, _F32, _P, _P]),
     "na_weight_norm_fwd": (ctypes.c_int, [_P, _P, _I64, _I64, _P, _P, _I32, _I64, _P]),
     "na_weight_norm_bwd": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _P, _P]),
     "na_sdf_input_fwd": (ctypes.c_int, [_PGRID, _P, _I64, _F32, _F32, _P, _I32, _I32, _P, _I32, _I64, _P]),

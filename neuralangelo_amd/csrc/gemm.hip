@@ -8,19 +8,17 @@
 //   split-K atomics (weight gradients, reduced over millions of points).
 // Tiles: 128x128x32 per 256-thread workgroup, each of the 4 waves owns a 64x64
 // sub-tile computed as 2x2 MFMA 32x32 blocks (bf16: v_mfma_f32_32x32x16_bf16,
-// fp32: v_mfma_f32_32x32x2_f32), operands staged through LDS.
+// fp32: the same instruction on three-way split operands), staged through LDS.
 //
 // Narrow layers (N <= 4: SDF head, colour output) use a wave-per-row kernel,
 // and weight normalisation (torch.nn.utils.weight_norm, dim=0) has its own
 // small kernels.
-#include "common.h"
+#include "mfma.h"
 
 #include <mutex>
 
 namespace na {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
 constexpr int GBM = 128, GBN = 128, GNT = 256;
 
@@ -1186,13 +1184,6 @@ enum PersistKind : int {
   PK_TAPS_BWD = 6,      // backward of the increments: C = tap rows, centre +=, shared rows, sums
 };
 
-// softplus_beta with a select for the linear region (no branch); ib = 1 / beta
-__device__ inline float softplus_sel(float v, float beta, float ib) {
-  const float z = v * beta;
-  const float r = fmaxf(v, 0.0f) + __logf(1.0f + __expf(-fabsf(z))) * ib;
-  return z > 20.0f ? v : r;
-}
-
 // Increment h = softplus(z0 + dz) - softplus(z0) and value y1 = softplus(z0 + dz)
 // for softplus(z) = ln(1 + exp(b z)) / b.  With a0 = b z0, u = b dz and the two
 // factors t0 = exp(-|a0|), e = exp(-|u|) in (0, 1], taking the larger exponent
@@ -1807,15 +1798,6 @@ gemm_bf16_nn_persist_kernel(GemmParams p) {
 // transposed (weight gradients; before, also too few parts of the sum): 256 x 136 over
 // 196,608 rows 427 -> 162 us, 256 x 280 over 28,800 rows 302 -> 58 us, 256 x 84 over 3,200
 // rows 380 -> 14 us.
-typedef __attribute__((ext_vector_type(8))) float f32x8_t;
-
-__device__ inline void split3(const f32x8_t& x, bf16x8_t (&h)[3]) {
-  h[0] = __builtin_convertvector(x, bf16x8_t);
-  const f32x8_t r = x - __builtin_convertvector(h[0], f32x8_t);
-  h[1] = __builtin_convertvector(r, bf16x8_t);
-  h[2] = __builtin_convertvector(r - __builtin_convertvector(h[1], f32x8_t), bf16x8_t);
-}
-
 constexpr int kF3BK = 32, kF3BM = 128;
 
 // One operand tile of R rows x 32 k, float32 chunks in registers.  Rows past the

@@ -332,6 +332,16 @@ def sdf_input(enc, points, cdt, k0p):
 def sdf_forward_nograd(enc, w, points):
     """SDF value only, no autograd state (sampling passes)."""
     P = points.shape[0]
+    table = enc.table_for_forward()
+    if table.dtype == w.cdt and _lib.call("na_sdf_value_supported", ctypes.byref(enc.desc),
+                                          _code(table), w.hidden):
+        sdf = torch.empty(P, 1, dtype=torch.float32, device=points.device)
+        vmin, vmax = enc.vol_range
+        _lib.call("na_sdf_value", ctypes.byref(enc.desc), _lib.ptr(points), P, float(vmin),
+                  float(vmax), _lib.ptr(table), _code(table), int(enc.active_levels),
+                  _lib.ptr(w.W0p), w.k0p, w.hidden, _lib.ptr(w.b0), _lib.ptr(w.ws), _lib.ptr(w.bs),
+                  float(SOFTPLUS_BETA), _lib.ptr(sdf), _s(points))
+        return sdf
     X0 = sdf_input(enc, points, w.cdt, w.k0p)
     H0 = torch.empty(P, w.hidden, dtype=w.cdt, device=points.device)
     gemm(X0, w.k0p, 0, w.W0p, w.k0p, 0, P, w.hidden, w.k0p, H0, w.hidden, bias=w.b0,
