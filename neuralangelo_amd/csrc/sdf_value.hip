@@ -252,6 +252,10 @@ static int launch_sdf_value(const na_grid_desc& d, const SdfValueParams& p, int6
 
 using namespace na;
 
+// The shapes with an instantiation: the presets' 16 levels of 4 or 8 features (a K of 64 or
+// 128, whole 16-wide steps, whose planes leave two workgroups' LDS per CU) and hidden
+// widths of four or eight 32-column waves.  There one launch was faster at each measured
+// count (64 points 12-16 us against 28-32, 131,072 points 1.3 to 1.7 times); other shapes take the three separate launches.
 extern "C" int na_sdf_value_supported(const na_grid_desc* d, int32_t dtype, int64_t N) {
   return d && d->n_levels == 16 && (d->n_features == 4 || d->n_features == 8) &&
          (dtype == NA_F32 || dtype == NA_BF16) && (N == 128 || N == 256);
