@@ -424,9 +424,11 @@ sdf_taps_input_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n, fl
 // removes most of the atomics.  What remains is bounded by the atomics' read-modify-write
 // of scattered entries (fine levels touch up to 27 corners of a box), so two lanes per
 // feature share a box and send neighbours in x together; the vector work that both
-// repeat is below a quarter of the time.  1,048,576 points, 8 features, bf16 rows: 3.33 ms
-// with one lane per feature and corner by corner, 2.90 ms; 65,536 points, 4 features,
-// float32: 261 us and 198 us.  When a level's cells spread wider than one cell
+// repeat is below a quarter of the time.  786,432 points, 8 features, bf16 rows: 3.33 ms
+// with one lane per feature and corner by corner, 2.90 ms; 49,152 points, 4 features,
+// float32: 261 us and 198 us.  The price is paid where samples lie so close that few
+// atomics remain: a dense step at the initial field takes 1.85 ms, 1.66 with one lane;
+// choosing per wave by whether its runs leave their cell did not win it back (1.84).  When a level's cells spread wider than one cell
 // (an epsilon larger than the finest active cell), that point falls back to
 // one atomic per point and corner.
 
