@@ -2214,7 +2214,9 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
   // made each tile's first stage wait for those operands: the tap product
   // 1.62 ms at 3.16 M rows, 1.28 ms now.)
   constexpr int kOperands = KIND == PK_DACT ? 8 : (KIND == PK_DELTA || KIND == PK_TAPS_FWD ? 16 : 0);
-  constexpr auto wait_code = [](int n) { return 0xF70 | (n & 15) | ((n >> 4) << 14); };
+  // A stage is read with 8 LDS reads per wave, which return in order: with at most 8
+  // outstanding (lgkmcnt), those of the stage before the last one have returned.
+  constexpr auto wait_code = [](int n) { return 0x870 | (n & 15) | ((n >> 4) << 14); };
   constexpr int kAhead = (kWsNS - 3) * LOADS;
   static_assert(kAhead + kOperands < 64, "stage waits");
   __shared__ __attribute__((aligned(16))) unsigned char smem[kWsNS * kWsStage * 2];
@@ -2285,11 +2287,12 @@ __global__ void __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) gemm_bf16_ws_kerne
   // workgroup waits for them before it ends.  With a fixed count of loads per
   // iteration the compiler's waits for the per-tile operand registers below
   // count exactly the stage loads issued after them.
-// One slot stays free: at a stage's barrier a wave's last reads of the previous stage may
+  // One slot stays free: at a stage's barrier a wave's last reads of the previous stage may
   // still be queued (the products that use them can come after the barrier), so the
-  // load issued there goes to the slot of the stage before that.  (A stage past the last
-  // tile reads no memory and writes its zeros at once, soon enough to overtake such
-  // reads; waiting for them at the barrier instead cost the tap product 7 %.)
+  // load issued there goes to the slot of the stage before that, whose reads the stage's wait
+  // has seen return.  (A stage past the last tile reads no memory and writes its zeros at
+  // once, soon enough to overtake queued reads; waiting for all reads at the barrier cost the
+  // tap product 7 %.)
 #pragma unroll
   for (int s = 0; s < kWsNS - 2; ++s) issue_next();
 
