@@ -1,5 +1,6 @@
 """The waits that staged kernels rely on, checked in the instructions of the built library: a
 missing one would show in results only now and then."""
+import heapq
 import re
 
 import pytest
@@ -37,3 +38,65 @@ def test_stationary_stage_slots(stationary):
         for reads, since in stages:
             assert reads == 8, name
             assert any(lgkm is not None and lgkm <= 8 for _, lgkm in since), name
+
+
+VMEM = re.compile(r"(global|buffer|flat)_(load|store|atomic)")
+
+
+def to_lds(c):
+    return c[2].endswith(" lds") or "load_lds" in c[1]
+
+
+def predecessors(code):
+    """Per instruction: the instructions that control can come from."""
+    by_address = {c[0]: i for i, c in enumerate(code)}
+    before = [[] for _ in code]
+    for i, (_, op, _, to) in enumerate(code):
+        if to in by_address:
+            before[by_address[to]].append(i)
+        if op not in ("s_branch", "s_endpgm") and i + 1 < len(code):
+            before[i + 1].append(i)
+    return before
+
+
+def fewest_after(code, at, behind):
+    """Fewest vector memory operations that a wave has issued, on any path to code[at], after
+    its last-but-`behind` stage load; None where no path holds so many stage loads."""
+    before = predecessors(code)
+    best, queue = {}, [(0, at, 0)]
+    while queue:
+        ops, i, stages = heapq.heappop(queue)
+        if best.setdefault((i, stages), ops) < ops:
+            continue
+        for j in before[i]:
+            n, s = ops, stages
+            if VMEM.match(code[j][1]):
+                if to_lds(code[j]):
+                    s += 1
+                    if s > behind:
+                        return ops
+                n += 1
+            if (j, s) not in best or best[j, s] > n:
+                best[j, s] = n
+                heapq.heappush(queue, (n, j, s))
+    return None
+
+
+def test_stationary_stage_arrival(stationary):
+    """A stage's load has landed at its barrier: memory operations complete in order, so the
+    wave may leave outstanding only as many as it has issued after that load, on every path.
+    Operand loads that are counted there must not be merged, dropped or moved past the wait."""
+    for name, code in stationary.items():
+        waves = int(re.search(r"ILi(\d)ELi\dELi\dE", name)[1])
+        slots, loads = (15, 1) if waves == 8 else (9, 2)
+        checked = 0
+        for i, (_, op, args, _) in enumerate(code):
+            if op != "s_waitcnt" or "s_barrier" not in [c[1] for c in code[i:i + 5]]:
+                continue
+            allowed = waits(args)[0]
+            if not allowed:
+                continue
+            issued = fewest_after(code, i, (slots - 3) * loads)
+            assert issued is not None and allowed <= issued, (name, i, allowed, issued)
+            checked += 1
+        assert checked >= int(re.search(r"ELi(\d)ELi\dE", name)[1]) - 1, name
