@@ -990,12 +990,13 @@ __device__ inline void nn_issue_stage(const bf16_t* __restrict__ X, int64_t ld, 
 }
 
 // Wait until at most `pending` of this wave's stage loads are outstanding
-// (4 load instructions per stage).  vmcnt is an immediate operand.
+// (4 load instructions per stage) and its LDS reads have returned: past the barrier that
+// follows, the slot they read is refilled.  vmcnt is an immediate operand.
 __device__ inline void nn_wait_stages(int pending) {
-  // gfx9 s_waitcnt immediate: vmcnt[3:0], expcnt[6:4] = 7, lgkmcnt[11:8] = 15
-  if (pending >= 2) __builtin_amdgcn_s_waitcnt(0xF70 | 8);
-  else if (pending == 1) __builtin_amdgcn_s_waitcnt(0xF70 | 4);
-  else __builtin_amdgcn_s_waitcnt(0xF70);
+  // gfx9 s_waitcnt immediate: vmcnt[3:0], expcnt[6:4] = 7, lgkmcnt[11:8] = 0
+  if (pending >= 2) __builtin_amdgcn_s_waitcnt(0x070 | 8);
+  else if (pending == 1) __builtin_amdgcn_s_waitcnt(0x070 | 4);
+  else __builtin_amdgcn_s_waitcnt(0x070);
 }
 
 __global__ void __launch_bounds__(GNT)
@@ -1121,14 +1122,15 @@ __device__ inline void persist_issue(const __amdgpu_buffer_rsrc_t ra, const __am
 }
 
 // Wait until at most `ahead` stages (LOADS instructions each) issued after the
-// one needed now are outstanding.  vmcnt is an immediate operand.
+// one needed now are outstanding and the wave's LDS reads have returned: past the barrier
+// that follows, the slot they read is refilled.  vmcnt is an immediate operand.
 template <int LOADS>
 __device__ inline void persist_wait(int ahead) {
   switch (ahead) {
-    case 0: __builtin_amdgcn_s_waitcnt(0xF70); break;
-    case 1: __builtin_amdgcn_s_waitcnt(0xF70 | (1 * LOADS)); break;
-    case 2: __builtin_amdgcn_s_waitcnt(0xF70 | (2 * LOADS)); break;
-    default: __builtin_amdgcn_s_waitcnt(0xF70 | (3 * LOADS)); break;
+    case 0: __builtin_amdgcn_s_waitcnt(0x070); break;
+    case 1: __builtin_amdgcn_s_waitcnt(0x070 | (1 * LOADS)); break;
+    case 2: __builtin_amdgcn_s_waitcnt(0x070 | (2 * LOADS)); break;
+    default: __builtin_amdgcn_s_waitcnt(0x070 | (3 * LOADS)); break;
   }
 }
 

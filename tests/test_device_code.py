@@ -100,3 +100,26 @@ def test_stationary_stage_arrival(stationary):
             assert issued is not None and allowed <= issued, (name, i, allowed, issued)
             checked += 1
         assert checked >= int(re.search(r"ELi(\d)ELi\dE", name)[1]) - 1, name
+
+
+@pytest.mark.parametrize("kernel", ["gemm_bf16_nn_kernel", "gemm_bf16_nn_persist_kernel",
+                                    "gemm_bf16_wgrad_kernel"])
+def test_refilled_stage_was_read(kernel):
+    """These kernels refill the slot of the stage before: its reads have returned when a wave
+    arrives at the barrier in front of the stage loads, by the wait ahead of it."""
+    for name, code in kernels(kernel).items():
+        before, stages = predecessors(code), set()
+        queue = [i for i, c in enumerate(code) if to_lds(c)]
+        seen = set(queue)
+        while queue:  # back from the stage loads to the barriers ahead of them
+            i = queue.pop()
+            if code[i][1] == "s_barrier":
+                stages.add(i)
+                continue
+            new = [j for j in before[i] if j not in seen]
+            seen.update(new)
+            queue += new
+        assert stages, name
+        for i in stages:
+            wait = [waits(c[2]) for c in code[max(i - 4, 0):i] if c[1] == "s_waitcnt"]
+            assert any(vm is not None and lgkm == 0 for vm, lgkm in wait), name
