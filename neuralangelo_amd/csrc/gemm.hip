@@ -1808,7 +1808,7 @@ constexpr int kF3BK = 32, kF3BM = 128;
 // products; what lies past the end of K is cleared by store().
 // TRANS = false: element (r, k) at X[r ld + k], a thread takes 8 k of NC rows, 64 apart.
 // TRANS = true: element (r, k) at X[k ld + r], threads t < R take 4 r x 8 k each (NC = 4);
-// QUADS: the operand's width is a multiple of 4 (else element by element).
+// QUADS: the operand's width is a multiple of 4 (else its last columns go one by one).
 template <int NC, int R, bool TRANS, bool QUADS>
 struct SplitLoader {
   float4 q[NC][2];  // TRANS: k row e of the thread's 8 at q[e / 2][e % 2]
@@ -1849,7 +1849,7 @@ struct SplitLoader {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float* s = row[0] + (k + (c + e < n ? c + e : 0)) * ld;
-        if constexpr (QUADS) {
+        if (QUADS || left >= 4) {
           q[e / 2][e % 2] = *reinterpret_cast<const float4*>(s);
         } else {
           q[e / 2][e % 2] = make_float4(left > 0 ? s[0] : 0.0f, left > 1 ? s[1] : 0.0f,
@@ -1903,7 +1903,7 @@ __device__ inline float f3_at(const float* __restrict__ X, int64_t ld, int64_t r
 // time, with 16-byte loads and stores.  F3_ATOMIC: a lane holds one column (rows in
 // registers), so an atomic instruction covers whole row segments.  F3_GENERAL: the
 // staged epilogue, for unaligned rows, widths that are not multiples of 8 and the
-// rare epilogue terms.
+// rare epilogue terms.  Each mode takes each operand layout it is launched with below.
 enum F3Mode : int { F3_ROWS, F3_ATOMIC, F3_GENERAL };
 
 __device__ inline float sum_lanes32(float v) {  // over the lanes that share lane >> 5
@@ -1948,7 +1948,7 @@ __device__ inline void f3_finish8(const EpiParams& e, int64_t m, int64_t col, fl
   }
 }
 
-template <bool TA, bool TB, int NB, int MODE>
+template <bool TA, bool TB, int NB, int MODE, bool QUADS>
 __global__ void __launch_bounds__(GNT, 2)
 gemm_f32_kernel(GemmParams p, int64_t parts) {
   constexpr int BM = kF3BM, BN = 32 * NB;
@@ -1975,8 +1975,8 @@ gemm_f32_kernel(GemmParams p, int64_t parts) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[j][r] = low[j][r] = 0.0f;
 
-  SplitLoader<TA ? 4 : BM / 64, BM, TA, MODE != F3_GENERAL> la;
-  SplitLoader<TB ? 4 : (BN + 63) / 64, BN, TB, MODE != F3_GENERAL> lb;
+  SplitLoader<TA ? 4 : BM / 64, BM, TA, QUADS> la;
+  SplitLoader<TB ? 4 : (BN + 63) / 64, BN, TB, QUADS> lb;
   // transposed tiles of 128 rows and up to 128 columns use one half of the threads each
   const int tb = TA && TB ? (tid + GNT / 2) & (GNT - 1) : tid;
   la.init((const float*)p.A, p.lda, m0, p.M, kbeg, tid);
@@ -2102,9 +2102,9 @@ gemm_f32_kernel(GemmParams p, int64_t parts) {
         if (n0 + c < p.N) atomic_add_f32(e.colsum + slot_offset(e.slots, e.slot_stride) + n0 + c, s_col[c]);
     }
   } else {
-    static_assert(MODE != F3_GENERAL || NB == 4, "the staged epilogue takes 64 columns at a time");
+    static_assert(MODE != F3_GENERAL || NB % 2 == 0, "the staged epilogue takes 64 columns at a time");
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
+    for (int half = 0; half < NB / 2; ++half) {
       f32x16_t part[1][2] = {{acc[2 * half], acc[2 * half + 1]}};
       gemm_epilogue<4, false>(p, smem, part, m0, n0, wave, half, wave, lane);
     }
@@ -3090,7 +3090,7 @@ static bool f32_rows_ok(const na_gemm_args* a) {
          (!a->r1_a || aligned16(a->r1_b)) && (!a->dact || rows8(a->dact_y, a->ld_dact, a->dact_dtype));
 }
 
-template <bool TA, bool TB, int MODE>
+template <bool TA, bool TB, int MODE, bool QUADS = MODE == F3_ATOMIC || (!TA && !TB)>
 static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
   // Split the sum over K where the output is added with atomics and no epilogue term
   // is nonlinear: two workgroups per CU, of at least 96 values each.  (The weight
@@ -3098,8 +3098,14 @@ static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
   // a million rows: 380 us at 3,200 rows, where 34 parts take 14.)
   const int64_t rows = ceil_div(p.M, (int64_t)kF3BM), blocks = ceil_div(p.N, (int64_t)32);
   int64_t cols = blocks <= 5 ? 1 : ceil_div(blocks, (int64_t)4), parts = 1;
+  // A transposed operand takes tiles of 64 columns (general), 64 or 128 (rows): its loader
+  // and the accumulators of 128 columns leave the general epilogue no registers.
+  // 200,000 x 256 x 136 with either operand transposed: 329 us on spilling 128-column tiles with
+  // the general epilogue, 158 to 170 here; 500 rows 40 and 15 us.
+  constexpr int kGeneralNB = TA || TB ? 2 : 4;
+  constexpr bool kEven = MODE == F3_ROWS && (TA || TB);
   if (MODE == F3_GENERAL) {
-    cols = ceil_div(blocks, (int64_t)4);
+    cols = ceil_div(blocks, (int64_t)kGeneralNB);
     if (a->split_k > 1) parts = a->split_k;
   } else if (MODE == F3_ATOMIC) {
     // transposed tiles of up to 96 columns load beside the 128 rows, with both
@@ -3112,7 +3118,8 @@ static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
     // narrower tiles where these would leave CUs idle
     while (rows * cols < 512 && cols * 2 <= blocks) cols *= 2;
   }
-  int nb = MODE == F3_GENERAL ? 4 : (int)ceil_div(blocks, cols);
+  int nb = MODE == F3_GENERAL ? kGeneralNB : (int)ceil_div(blocks, cols);
+  if (kEven) nb = nb <= 2 ? 2 : 4;
   cols = ceil_div(blocks, (int64_t)nb);
   p.k_chunk = ceil_div(ceil_div(p.K, parts < 1 ? 1 : parts), (int64_t)kF3BK) * kF3BK;
   if (p.k_chunk < kF3BK) p.k_chunk = kF3BK;
@@ -3121,15 +3128,18 @@ static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
   const int64_t blocks_all = units < 64 ? units * cols : ceil_div(units, (int64_t)8) * 8 * cols;
   NA_CHECK_ARG(blocks_all < 0x7fffffffLL, "GEMM grid too large");
   const dim3 grid((unsigned)blocks_all);
-#define NA_F3(NB) hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, NB, MODE>), grid, dim3(GNT), 0, s, p, parts)
+#define NA_F3(NB) hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, NB, MODE, QUADS>), grid, dim3(GNT), 0, s, p, parts)
   if constexpr (MODE == F3_GENERAL) {
-    NA_F3(4);
+    NA_F3(kGeneralNB);
   } else if constexpr (MODE == F3_ATOMIC) {
     switch (nb) {
       case 1: NA_F3(1); break;
       case 2: NA_F3(2); break;
       default: NA_F3(3); break;
     }
+  } else if constexpr (kEven) {
+    if (nb == 2) NA_F3(2);
+    else NA_F3(4);
   } else {
     switch (nb) {
       case 1: NA_F3(1); break;
@@ -3151,9 +3161,12 @@ static int run_gemm_f32(const na_gemm_args* a, const GemmParams& p, hipStream_t 
     return plain ? launch_gemm_f32<true, true, F3_ATOMIC>(a, p, s)
                  : launch_gemm_f32<true, true, F3_GENERAL>(a, p, s);
   }
-  if (a->trans_a) return launch_gemm_f32<true, false, F3_GENERAL>(a, p, s);
-  if (a->trans_b) return launch_gemm_f32<false, true, F3_GENERAL>(a, p, s);
-  return f32_rows_ok(a) ? launch_gemm_f32<false, false, F3_ROWS>(a, p, s)
+  const bool rows = f32_rows_ok(a);
+  if (a->trans_a)
+    return rows ? launch_gemm_f32<true, false, F3_ROWS>(a, p, s) : launch_gemm_f32<true, false, F3_GENERAL>(a, p, s);
+  if (a->trans_b)
+    return rows ? launch_gemm_f32<false, true, F3_ROWS>(a, p, s) : launch_gemm_f32<false, true, F3_GENERAL>(a, p, s);
+  return rows ? launch_gemm_f32<false, false, F3_ROWS>(a, p, s)
                         : launch_gemm_f32<false, false, F3_GENERAL>(a, p, s);
 }
 

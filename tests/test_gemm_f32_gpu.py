@@ -87,3 +87,29 @@ def test_values_that_do_not_split(ta, tb, N):
     fin = ref.isfinite()
     assert torch.equal(C[C.isinf()].sign().double(), ref[ref.isinf()].sign())
     assert ((C.double() - ref).abs()[fin] <= bound(A, B, K)[fin]).all()
+
+
+@pytest.mark.parametrize("ta, tb", [(1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M, N, K", [(129, 256, 68), (300, 40, 100), (70, 70, 36)])
+def test_epilogue_terms_of_transposed_operands(M, N, K, ta, tb):
+    """Tiles of 64 and 128 columns, and widths that only the staged epilogue takes."""
+    g = torch.Generator().manual_seed(M)
+    A, a, lda = operand(M, K, ta, g, 0.1)
+    B, b, ldb = operand(N, K, tb, g, 0.1)
+    bias = torch.randn(N, generator=g).cuda()
+    z = A.double() @ B.double().t()
+    err = bound(A, B, K) + 2.0 ** -23 * (z + bias.double()).abs()
+    C = torch.empty(M, N, device="cuda")
+    Fn.gemm(a, lda, ta, b, ldb, tb, M, N, K, C, N, bias=bias, act=NA_ACT_SOFTPLUS)
+    ref = torch.nn.functional.softplus(z + bias.double(), beta=100)
+    assert ((C.double() - ref).abs() <= err + 1e-8 + 2.0 ** -22 * ref.abs()).all()
+    y = torch.rand(M, N, generator=g).cuda() - 0.3
+    r1a, r1b = torch.randn(M, generator=g).cuda(), torch.randn(N, generator=g).cuda()
+    r1 = r1a.double()[:, None] * r1b.double()
+    cs = torch.ones(N, device="cuda")
+    Fn.gemm(a, lda, ta, b, ldb, tb, M, N, K, C, N, dact=NA_ACT_RELU, dact_y=y, ld_dact=N, r1_a=r1a,
+            r1_b=r1b, colsum=cs)
+    v = (z + r1) * (y > 0)
+    e = err + 2.0 ** -22 * r1.abs() + 2.0 ** -23 * z.abs()
+    assert ((C.double() - v).abs() <= e).all()
+    assert ((cs.double() - 1 - v.sum(0)).abs() <= e.sum(0) + M * 2.0 ** -23 * (1 + v.abs().sum(0))).all()
