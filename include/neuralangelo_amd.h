@@ -133,7 +133,9 @@ int na_hashgrid_bwd(const na_grid_desc* desc, const float* x, int64_t n,
  * epilogue, in order: v += bias[n]; v = act(v); v += r1_a[m]*r1_b[n];
  *   v *= act'(dact_y[m*ld_dact+n]) (derivative expressed through the
  *   activation's output y); colsum[n] += v (atomic); store/accumulate v.
- * A and B share in_dtype (NA_F32: fp32 MFMA, NA_BF16: bf16 MFMA); the
+ * A and B share in_dtype (NA_F32: bf16 MFMA on operands split into three bf16 parts,
+ * which hold a float32 value exactly from 2^-109 up (smaller ones lose their last
+ * bits) and whose products reach float32 accuracy; NA_BF16: bf16 MFMA); the
  * accumulation is fp32.  K and the leading dimensions must be multiples of 8
  * (bf16) or 4 (fp32) and the pointers 16-byte aligned. */
 typedef struct na_gemm_args {
@@ -177,11 +179,13 @@ typedef struct na_gemm_args {
   int64_t zc_rows;
   const float* head_w;
   float* head_out;
-  /* optional workspace of the weight-gradient path (bf16, trans_a = trans_b = 1,
+  /* optional workspace of the weight-gradient path (trans_a = trans_b = 1,
    * atomic epilogue, no epilogue terms): each row split stores its partial
    * product here and one more launch adds the splits into C in split order
    * (no atomics; the result does not depend on scheduling).  wg_partials_len
-   * floats, at least na_gemm_wgrad_workspace(args); NULL or shorter = atomics. */
+   * floats, at least na_gemm_wgrad_workspace(args); NULL or shorter = atomics,
+   * from split_k parts (float32: 1 adds once to each output) or from the bf16
+   * path's own split. */
   float* wg_partials;
   int64_t wg_partials_len;
 } na_gemm_args;
@@ -266,7 +270,8 @@ int na_taps_increment_bwd_slots(const void* D, int64_t ld_d, int64_t M, int64_t 
 int na_gemm_wgrad_static(const na_gemm_args* args, na_stream_t stream);
 
 /* Floats of wg_partials that na_gemm's weight-gradient path uses for these
- * arguments (0 when another path runs them; NA_ERR_ARGUMENT for a NULL args). */
+ * arguments (0 when another path runs them, or a float32 sum in one part, which adds
+ * once to each output; NA_ERR_ARGUMENT for a NULL args). */
 int64_t na_gemm_wgrad_workspace(const na_gemm_args* args);
 
 /* out[n] += sum_m X[m*ld + n] (fp32 accumulation, X of x_dtype): the bias gradient

@@ -64,6 +64,7 @@ struct GemmParams {
   const void* B;
   int64_t ldb;
   int64_t k_chunk;
+  float* part;  // weight gradients: partial products [part of K][M][N], or null
   EpiParams e;
 };
 
@@ -2049,14 +2050,17 @@ gemm_f32_kernel(GemmParams p, int64_t parts) {
   }
 
   if constexpr (MODE == F3_ATOMIC) {
-    float* C = (float*)p.e.C;
+    float* C = p.part ? p.part + unit / rows * p.M * p.N : (float*)p.e.C;
+    const int64_t ldc = p.part ? p.N : p.e.ldc;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       const int64_t n = n0 + j * 32 + (lane & 31);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t m = m0 + wave * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (m < p.M && n < p.N) atomic_add_f32(C + m * p.e.ldc + n, acc[j][r]);
+        if (m >= p.M || n >= p.N) continue;
+        if (p.part) C[m * ldc + n] = acc[j][r];
+        else atomic_add_f32(C + m * ldc + n, acc[j][r]);
       }
     }
   } else if constexpr (MODE == F3_ROWS) {
@@ -3036,6 +3040,16 @@ static WgradPlan wgrad_plan(const na_gemm_args* a) {
   return w;
 }
 
+static int launch_wgrad_reduce(const float* part, int64_t splits, int64_t N, int64_t K, float* C,
+                               int64_t ldc, hipStream_t s) {
+  const int64_t blocks = ceil_div(N * K, (int64_t)64);
+  NA_CHECK_ARG(blocks < 0x7fffffffLL, "weight-gradient output too large");
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, part, splits, N, K,
+                     C, ldc);
+  NA_CHECK_LAUNCH();
+  return NA_OK;
+}
+
 static int launch_wgrad(const na_gemm_args* a, hipStream_t s) {
   const WgradPlan w = wgrad_plan(a);
   const int64_t bk = 64 * w.kb;
@@ -3056,14 +3070,7 @@ static int launch_wgrad(const na_gemm_args* a, hipStream_t s) {
   else NA_WG(5);
 #undef NA_WG
   NA_CHECK_LAUNCH();
-  if (use_part) {
-    const int64_t blocks = ceil_div(w.No * w.Ko, (int64_t)64);
-    NA_CHECK_ARG(blocks < 0x7fffffffLL, "weight-gradient output too large");
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, part, w.splits,
-                       w.No, w.Ko, C, a->ldc);
-    NA_CHECK_LAUNCH();
-  }
-  return NA_OK;
+  return use_part ? launch_wgrad_reduce(part, w.splits, w.No, w.Ko, C, a->ldc, s) : NA_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -3090,14 +3097,36 @@ static bool f32_rows_ok(const na_gemm_args* a) {
          (!a->r1_a || aligned16(a->r1_b)) && (!a->dact || rows8(a->dact_y, a->ld_dact, a->dact_dtype));
 }
 
-template <bool TA, bool TB, int MODE, bool QUADS = MODE == F3_ATOMIC || (!TA && !TB)>
+// Float32 weight gradients: a sum over K that adds to C, without epilogue terms.
+static bool f32_wgrad_ok(const na_gemm_args* a) {
+  return a->in_dtype == NA_F32 && a->trans_a && a->trans_b && a->epilogue == NA_EPI_ATOMIC &&
+         a->c_dtype == NA_F32 && !a->bias && !a->act && !a->dact && !a->r1_a && !a->colsum &&
+         !a->z_out && !a->zc && !a->head_w;
+}
+
+// Column tiles of f32_wgrad_ok products: up to 96 columns load beside the 128 rows, with both
+// accumulators in registers.
+static int64_t f32_wgrad_cols(const na_gemm_args* a) { return ceil_div(a->N, (int64_t)96); }
+
+// Parts of the sum when a workspace takes them: as many as two workgroups per CU hold at
+// once, counted per XCD (a unit's column tiles stay on one), of at least 96 values each.  One
+// part, or one per 2048 rows, leaves most CUs idle below half a million rows: 256 x 84 over 3,200
+// rows 380 us, in 34 parts 15.  A part more than fits starts a second round: 256 x 256
+// over 196,608 rows 354 us in 86 parts, 234 in 84.
+static int64_t f32_wgrad_parts(const na_gemm_args* a) {
+  const int64_t units = 8 * (64 / f32_wgrad_cols(a));
+  const int64_t parts = std::max<int64_t>(
+      1, std::min(units / ceil_div(a->M, (int64_t)kF3BM), ceil_div(a->K, (int64_t)96)));
+  const int64_t chunk = ceil_div(ceil_div(a->K, parts), (int64_t)kF3BK) * kF3BK;
+  return a->K == 0 ? 1 : ceil_div(a->K, chunk);
+}
+
+template <bool TA, bool TB, int MODE, bool QUADS = !TA && !TB>
 static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
-  // Split the sum over K where the output is added with atomics and no epilogue term
-  // is nonlinear: two workgroups per CU, of at least 96 values each.  (The weight
-  // gradients ask for a part per 2048 rows, which leaves most CUs idle below half
-  // a million rows: 380 us at 3,200 rows, where 34 parts take 14.)
   const int64_t rows = ceil_div(p.M, (int64_t)kF3BM), blocks = ceil_div(p.N, (int64_t)32);
-  int64_t cols = blocks <= 5 ? 1 : ceil_div(blocks, (int64_t)4), parts = 1;
+  int64_t cols = blocks <= 5 ? 1 : ceil_div(blocks, (int64_t)4);
+  int64_t parts = a->split_k > 1 ? a->split_k : 1;
+  p.part = nullptr;
   // A transposed operand takes tiles of 64 columns (general), 64 or 128 (rows): its loader
   // and the accumulators of 128 columns leave the general epilogue no registers.
   // 200,000 x 256 x 136 with either operand transposed: 329 us on spilling 128-column tiles with
@@ -3106,14 +3135,13 @@ static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
   constexpr bool kEven = MODE == F3_ROWS && (TA || TB);
   if (MODE == F3_GENERAL) {
     cols = ceil_div(blocks, (int64_t)kGeneralNB);
-    if (a->split_k > 1) parts = a->split_k;
   } else if (MODE == F3_ATOMIC) {
-    // transposed tiles of up to 96 columns load beside the 128 rows, with both
-    // accumulators in registers
-    cols = ceil_div(blocks, (int64_t)3);
-    const int64_t most = ceil_div(p.K, (int64_t)96);
-    parts = ceil_div((int64_t)512, rows * cols);
-    if (parts > most) parts = most;
+    cols = f32_wgrad_cols(a);
+    const int64_t n = f32_wgrad_parts(a);
+    if (a->wg_partials && n > 1 && a->wg_partials_len >= n * a->M * a->N) {
+      parts = n;
+      p.part = a->wg_partials;
+    }
   } else {
     // narrower tiles where these would leave CUs idle
     while (rows * cols < 512 && cols * 2 <= blocks) cols *= 2;
@@ -3151,15 +3179,14 @@ static int launch_gemm_f32(const na_gemm_args* a, GemmParams p, hipStream_t s) {
   }
 #undef NA_F3
   NA_CHECK_LAUNCH();
-  return NA_OK;
+  return p.part ? launch_wgrad_reduce(p.part, parts, p.M, p.N, (float*)p.e.C, p.e.ldc, s) : NA_OK;
 }
 
 static int run_gemm_f32(const na_gemm_args* a, const GemmParams& p, hipStream_t s) {
   if (a->trans_a && a->trans_b) {
-    const bool plain = a->epilogue == NA_EPI_ATOMIC && !a->bias && !a->act && !a->dact && !a->r1_a &&
-                       !a->colsum && a->M % 4 == 0 && a->N % 4 == 0;
-    return plain ? launch_gemm_f32<true, true, F3_ATOMIC>(a, p, s)
-                 : launch_gemm_f32<true, true, F3_GENERAL>(a, p, s);
+    if (!f32_wgrad_ok(a)) return launch_gemm_f32<true, true, F3_GENERAL>(a, p, s);
+    return a->M % 4 == 0 && a->N % 4 == 0 ? launch_gemm_f32<true, true, F3_ATOMIC, true>(a, p, s)
+                                          : launch_gemm_f32<true, true, F3_ATOMIC, false>(a, p, s);
   }
   const bool rows = f32_rows_ok(a);
   if (a->trans_a)
@@ -3410,7 +3437,12 @@ extern "C" int na_taps_increment_bwd_slots(const void* D, int64_t ld_d, int64_t 
 
 extern "C" int64_t na_gemm_wgrad_workspace(const na_gemm_args* a) {
   NA_CHECK_ARG(a != nullptr, "args is null");
-  if (a->M <= 0 || a->N <= 0 || a->K <= 0 || !wgrad_ok(a)) return 0;
+  if (a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
+  if (f32_wgrad_ok(a)) {
+    const int64_t parts = f32_wgrad_parts(a);
+    return parts > 1 ? parts * a->M * a->N : 0;
+  }
+  if (!wgrad_ok(a)) return 0;
   const WgradPlan w = wgrad_plan(a);
   return w.splits * w.No * w.Ko;
 }

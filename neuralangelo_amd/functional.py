@@ -174,18 +174,12 @@ def _t(W):
     return W.t().contiguous()
 
 
-def _split_for(rows):
-    """split-K factor for weight-gradient GEMMs reducing over `rows` points."""
-    return max(1, min(512, rows // 2048))
-
-
 def linear_weight_grad(dpre, X, ldx, K, dW):
     """dW[n, k] += sum_m dpre[m, n] X[m, k]  (dpre [M, N] contiguous)."""
     M, N = dpre.shape
     if M == 0:
         return
-    gemm(dpre, N, 1, X, ldx, 1, N, K, M, dW, dW.stride(0), epilogue=NA_EPI_ATOMIC,
-         split_k=_split_for(M))
+    gemm(dpre, N, 1, X, ldx, 1, N, K, M, dW, dW.stride(0), epilogue=NA_EPI_ATOMIC)
 
 
 def act_grad(dy, y, act, out_dtype, colsum=None, n_cols=None, slots=(1, 0)):

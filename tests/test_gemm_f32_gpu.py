@@ -113,3 +113,36 @@ def test_epilogue_terms_of_transposed_operands(M, N, K, ta, tb):
     e = err + 2.0 ** -22 * r1.abs() + 2.0 ** -23 * z.abs()
     assert ((C.double() - v).abs() <= e).all()
     assert ((cs.double() - 1 - v.sum(0)).abs() <= e.sum(0) + M * 2.0 ** -23 * (1 + v.abs().sum(0))).all()
+
+
+@pytest.mark.parametrize("rows, N, K", [(500, 64, 36), (3200, 256, 84), (20001 * 4, 90, 131)])
+def test_weight_gradients_repeat(rows, N, K):
+    """With the workspace the parts of the sum add up in order: the same bits on every call."""
+    g = torch.Generator().manual_seed(rows)
+    D, dpre, ldd = operand(N, rows, 1, g)
+    X, x, ldx = operand(K, rows, 1, g)
+    out = []
+    for _ in range(4):
+        dW = torch.full((N, K), 0.25, device="cuda")
+        Fn.gemm(dpre, ldd, 1, x, ldx, 1, N, K, rows, dW, K, epilogue=NA_EPI_ATOMIC)
+        out.append(dW)
+    assert all(torch.equal(o, out[0]) for o in out[1:])
+    ref = D.double() @ X.double().t()
+    slack = 600 * 2.0 ** -24 * (ref.abs() + 0.25 + (D.double().abs() @ X.double().abs().t()))
+    assert ((out[0].double() - 0.25 - ref).abs() <= bound(D, X, rows) + slack).all()
+
+
+def test_split_k_of_one_is_one_addition():
+    """Without a workspace the caller's split_k holds: one part adds once to each output."""
+    rows, N, K = 3200, 256, 84
+    g = torch.Generator().manual_seed(1)
+    D, dpre, ldd = operand(N, rows, 1, g)
+    X, x, ldx = operand(K, rows, 1, g)
+    out = []
+    for _ in range(4):
+        dW = torch.zeros(N, K, device="cuda")
+        Fn.gemm(dpre, ldd, 1, x, ldx, 1, N, K, rows, dW, K, epilogue=NA_EPI_ATOMIC,
+                wgrad_partials=False)
+        out.append(dW)
+    assert all(torch.equal(o, out[0]) for o in out[1:])
+    assert ((out[0].double() - D.double() @ X.double().t()).abs() <= bound(D, X, rows)).all()
