@@ -183,9 +183,9 @@ typedef struct na_gemm_args {
    * atomic epilogue, no epilogue terms): each row split stores its partial
    * product here and one more launch adds the splits into C in split order
    * (no atomics; the result does not depend on scheduling).  wg_partials_len
-   * floats, at least na_gemm_wgrad_workspace(args); NULL or shorter = atomics,
-   * from split_k parts (float32: 1 adds once to each output) or from the bf16
-   * path's own split. */
+   * floats, at least na_gemm_wgrad_workspace(args) (bf16) or
+   * na_gemm_f32_wgrad_workspace(args); NULL or shorter = atomics, from the bf16 path's
+   * own split or, float32, from split_k parts (1 adds once to each output). */
   float* wg_partials;
   int64_t wg_partials_len;
 } na_gemm_args;
@@ -270,9 +270,10 @@ int na_taps_increment_bwd_slots(const void* D, int64_t ld_d, int64_t M, int64_t 
 int na_gemm_wgrad_static(const na_gemm_args* args, na_stream_t stream);
 
 /* Floats of wg_partials that na_gemm's weight-gradient path uses for these
- * arguments (0 when another path runs them, or a float32 sum in one part, which adds
- * once to each output; NA_ERR_ARGUMENT for a NULL args). */
+ * arguments (0 when another path runs them; NA_ERR_ARGUMENT for a NULL args): bf16
+ * products, and float32 ones (0 also for a sum in one part). */
 int64_t na_gemm_wgrad_workspace(const na_gemm_args* args);
+int64_t na_gemm_f32_wgrad_workspace(const na_gemm_args* args);
 
 /* out[n] += sum_m X[m*ld + n] (fp32 accumulation, X of x_dtype): the bias gradient
  * of a linear layer from its pre-activation gradient (torch.nn.Linear backward,

@@ -98,6 +98,7 @@ _SIGNATURES = {
     "na_gemm": (ctypes.c_int, [_PGEMM, _P]),
     "na_gemm_slots": (ctypes.c_int, [_PGEMM, _I32, _I64, _P]),
     "na_gemm_wgrad_workspace": (ctypes.c_int64, [_PGEMM]),
+    "na_gemm_f32_wgrad_workspace": (ctypes.c_int64, [_PGEMM]),
     "na_gemm_wgrad_static": (ctypes.c_int, [_PGEMM, _P]),
     "na_taps_increment_fwd": (ctypes.c_int, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _P,
                                              _F32, _P, _P, _P]),

@@ -3437,14 +3437,16 @@ extern "C" int na_taps_increment_bwd_slots(const void* D, int64_t ld_d, int64_t 
 
 extern "C" int64_t na_gemm_wgrad_workspace(const na_gemm_args* a) {
   NA_CHECK_ARG(a != nullptr, "args is null");
-  if (a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
-  if (f32_wgrad_ok(a)) {
-    const int64_t parts = f32_wgrad_parts(a);
-    return parts > 1 ? parts * a->M * a->N : 0;
-  }
-  if (!wgrad_ok(a)) return 0;
+  if (a->M <= 0 || a->N <= 0 || a->K <= 0 || !wgrad_ok(a)) return 0;
   const WgradPlan w = wgrad_plan(a);
   return w.splits * w.No * w.Ko;
+}
+
+extern "C" int64_t na_gemm_f32_wgrad_workspace(const na_gemm_args* a) {
+  NA_CHECK_ARG(a != nullptr, "args is null");
+  if (a->M <= 0 || a->N <= 0 || a->K <= 0 || !f32_wgrad_ok(a)) return 0;
+  const int64_t parts = f32_wgrad_parts(a);
+  return parts > 1 ? parts * a->M * a->N : 0;
 }
 
 extern "C" int na_gemm(const na_gemm_args* a, na_stream_t stream) {

@@ -105,7 +105,8 @@ def gemm(A, lda, trans_a, B, ldb, trans_b, M, N, K, C, ldc, epilogue=NA_EPI_STOR
         a.head_w, a.head_out = head_w.data_ptr(), head_out.data_ptr()
     ws = None
     if wgrad_partials and epilogue == NA_EPI_ATOMIC:
-        n = _lib.call("na_gemm_wgrad_workspace", ctypes.byref(a))
+        n = _lib.call("na_gemm_wgrad_workspace" if a.in_dtype == _lib.NA_BF16 else
+                      "na_gemm_f32_wgrad_workspace", ctypes.byref(a))
         if n > 0:
             ws = torch.empty(n, dtype=torch.float32, device=C.device)
             a.wg_partials, a.wg_partials_len = ws.data_ptr(), n
