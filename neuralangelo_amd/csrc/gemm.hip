@@ -3208,7 +3208,8 @@ act_grad_vec_kernel(const TD* __restrict__ dy, int64_t ld_dy, const TY* __restri
                     int64_t M, int64_t N, int act, float beta, TO* __restrict__ out, int64_t ld_out,
                     float* __restrict__ colsum, int slots, int64_t slot_stride,
                     int64_t rows_per_block) {
-  __shared__ float red[256 * 8];
+  constexpr int kPitch = 257;
+  __shared__ float red[8 * kPitch];
   const int cpr = (int)(N / 8);
   const int c = threadIdx.x % cpr, r = threadIdx.x / cpr, lanes = 256 / cpr;
   const int64_t m0 = (int64_t)blockIdx.x * rows_per_block;
@@ -3246,16 +3247,15 @@ act_grad_vec_kernel(const TD* __restrict__ dy, int64_t ld_dy, const TY* __restri
     }
   }
   if (colsum) {
+    // consecutive columns leave from consecutive lanes, a request per cache line (8 columns a
+    // lane made eight requests of it, which queue at a single copy of the sums)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) red[k * 256 + threadIdx.x] = cs[k];
+    for (int k = 0; k < 8; ++k) red[k * kPitch + threadIdx.x] = cs[k];
     __syncthreads();
-    if (r == 0) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        float s = 0.0f;
-        for (int q = 0; q < lanes; ++q) s += red[k * 256 + q * cpr + c];
-        atomic_add_f32(colsum + slot_offset(slots, slot_stride) + 8 * c + k, s);
-      }
+    for (int n = threadIdx.x; n < N; n += 256) {
+      float s = 0.0f;
+      for (int q = 0; q < lanes; ++q) s += red[(n & 7) * kPitch + q * cpr + n / 8];
+      atomic_add_f32(colsum + slot_offset(slots, slot_stride) + n, s);
     }
   }
 }
