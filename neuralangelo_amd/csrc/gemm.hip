@@ -780,8 +780,10 @@ narrow_bwd_vec_kernel(const TX* __restrict__ X, int64_t ldx, int64_t M, int64_t 
     }
   }
   }
-  // combine the two half-waves (same k ranges), then the waves of the
-  // workgroup through LDS; one atomic per element leaves the workgroup
+  // Combine the two half-waves (same k ranges), then the waves of the workgroup through
+  // LDS, where each thread sums and adds single elements: one atomic per element, consecutive
+  // elements from consecutive lanes.  (Summed in the first wave's registers, eight
+  // neighbours a lane, four outputs spilled 100 registers and every request covered 4 bytes.)
 #pragma unroll
   for (int n = 0; n < NM; ++n) {
     gb[n] += __shfl_xor(gb[n], 32);
@@ -794,65 +796,39 @@ narrow_bwd_vec_kernel(const TX* __restrict__ X, int64_t ldx, int64_t M, int64_t 
   for (int c = 0; c < KC; ++c)
 #pragma unroll
     for (int e = 0; e < 8; ++e) cs[c][e] += __shfl_xor(cs[c][e], 32);
-  constexpr int PER = (NM + 1) * KC * 256 + NM;  // partials of one wave
+  constexpr int KP = KC * 256, PER = (NM + 1) * KP + NM;  // partials of one wave
   constexpr int WPG = NarrowBwdCfg<NM>::WPG;
-  __shared__ float red[(WPG - 1) * PER];
-  const int wv = threadIdx.x >> 6;
-  if (wv > 0 && half == 0) {
-    float* r = red + (wv - 1) * PER;
+  __shared__ float red[WPG * PER];
+  if (half == 0) {
+    float* r = red + (threadIdx.x >> 6) * PER;
 #pragma unroll
     for (int n = 0; n < NM; ++n)
 #pragma unroll
       for (int c = 0; c < KC; ++c)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) r[(n * KC + c) * 256 + 8 * hl + e] = gw[n][c][e];
+        for (int e = 0; e < 8; ++e) r[n * KP + 256 * c + 8 * hl + e] = gw[n][c][e];
 #pragma unroll
     for (int c = 0; c < KC; ++c)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[(NM * KC + c) * 256 + 8 * hl + e] = cs[c][e];
+      for (int e = 0; e < 8; ++e) r[NM * KP + 256 * c + 8 * hl + e] = cs[c][e];
     if (hl == 0)
 #pragma unroll
-      for (int n = 0; n < NM; ++n) r[(NM + 1) * KC * 256 + n] = gb[n];
+      for (int n = 0; n < NM; ++n) r[(NM + 1) * KP + n] = gb[n];
   }
   __syncthreads();
-  if (wv == 0 && half == 0) {
+  const int64_t so = slot_offset(slots, slot_stride);
+  for (int i = threadIdx.x; i < PER; i += 64 * WPG) {
+    // row n < NM: dW; n = NM: column sums of dX; the rest: db
+    const int n = i / KP, k = i % KP;
+    float* dst;
+    if (n < NM) dst = n < N && k < K ? dW + so + n * K + k : nullptr;
+    else if (n == NM) dst = dX && dx_colsum && k < K ? dx_colsum + so + k : nullptr;
+    else dst = k < N ? db + so + k : nullptr;
+    if (!dst) continue;
+    float v = 0.0f;
 #pragma unroll
-    for (int q = 0; q < WPG - 1; ++q) {
-      const float* r = red + q * PER;
-#pragma unroll
-      for (int n = 0; n < NM; ++n)
-#pragma unroll
-        for (int c = 0; c < KC; ++c)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) gw[n][c][e] += r[(n * KC + c) * 256 + 8 * hl + e];
-#pragma unroll
-      for (int c = 0; c < KC; ++c)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) cs[c][e] += r[(NM * KC + c) * 256 + 8 * hl + e];
-#pragma unroll
-      for (int n = 0; n < NM; ++n) gb[n] += r[(NM + 1) * KC * 256 + n];
-    }
-    const int64_t so = slot_offset(slots, slot_stride);
-    for (int n = 0; n < N; ++n) {
-#pragma unroll
-      for (int c = 0; c < KC; ++c)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int64_t k = 8 * hl + 256 * c + e;
-          if (k < K) atomic_add_f32(dW + so + n * K + k, gw[n][c][e]);
-        }
-    }
-    if (dX && dx_colsum) {
-#pragma unroll
-      for (int c = 0; c < KC; ++c)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int64_t k = 8 * hl + 256 * c + e;
-          if (k < K) atomic_add_f32(dx_colsum + so + k, cs[c][e]);
-        }
-    }
-    if (hl == 0)
-      for (int n = 0; n < N; ++n) atomic_add_f32(db + so + n, gb[n]);
+    for (int q = 0; q < WPG; ++q) v += red[q * PER + i];
+    atomic_add_f32(dst, v);
   }
 }
 

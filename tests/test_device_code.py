@@ -5,7 +5,7 @@ import re
 
 import pytest
 
-from device_code import kernels, waits
+from device_code import kernels, resources, waits
 
 
 @pytest.fixture(scope="module")
@@ -123,3 +123,10 @@ def test_refilled_stage_was_read(kernel):
         for i in stages:
             wait = [waits(c[2]) for c in code[max(i - 4, 0):i] if c[1] == "s_waitcnt"]
             assert any(vm is not None and lgkm == 0 for vm, lgkm in wait), name
+
+
+def test_narrow_backward_keeps_its_sums_in_registers():
+    """No variant of the narrow layer's backward spills (its tail once held every partial sum
+    of a workgroup in one wave)."""
+    for name, r in resources("narrow_bwd_vec_kernel").items():
+        assert r["vgpr_spill_count"] == 0 and r["private_segment_fixed_size"] == 0, name
