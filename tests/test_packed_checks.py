@@ -3,6 +3,7 @@ raised before a kernel is launched)."""
 import pytest
 import torch
 
+from neuralangelo_amd import _lib
 from neuralangelo_amd import functional as Fn
 
 
@@ -26,3 +27,11 @@ def test_valid_offsets_pass_the_checks():
     product path then refuses to run without the GPU."""
     with pytest.raises(RuntimeError, match="GPU"):
         Fn.check_offsets(torch.tensor([0, 0, 3, 3, 7], dtype=torch.int32), 7)
+
+
+def test_hier_resample_refuses_more_rays_than_a_launch_holds():
+    """Checked before any GPU call, like the other sizes."""
+    lib = _lib.load()
+    p = 0x1000  # not dereferenced: the size check comes first
+    st = lib.na_hier_resample(p, p, 2 ** 28, 64, 64.0, 16, p, p, p, p, None)
+    assert st == _lib.NA_ERR_ARGUMENT and "too many rays" in _lib.last_error()

@@ -300,3 +300,14 @@ def test_hierarchical_merge_order(cuda, R, N, Nf, rows):
                 want, at, j = fr[j], int(pf[r, j]), j + 1
             got = float(merged[r, k])
             assert at == k and (got == want or (got != got and want != want)), (r, k)
+
+
+@pytest.mark.parametrize("R, N, Nf", [(16384, 4, 4), (16385, 4, 4), (16385, 5, 4), (131072, 2, 1)])
+def test_hierarchical_round_of_few_samples(cuda, R, N, Nf):
+    """Many rays of few samples go by lane, others by wave: the same bits for every ray."""
+    g = torch.Generator().manual_seed(R + N)
+    d = (torch.rand(R, N, generator=g) * 2 + 2).sort(dim=1).values.to(cuda)
+    s = (d - 3.0) * -0.7 + 0.05 * torch.randn(R, N, generator=g).to(cuda)
+    got = nerf_util.hierarchical_round(d, s, 64.0, Nf)
+    ref = [nerf_util.hierarchical_round(d[k:k + 8000], s[k:k + 8000], 64.0, Nf) for k in range(0, R, 8000)]
+    assert all(torch.equal(a, torch.cat(b)) for a, b in zip(got, zip(*ref)))
