@@ -44,9 +44,15 @@ __device__ inline void chunk_level(int levels, int64_t& chunk, int& level) {
   chunk = (int64_t)(slot / (uint32_t)levels) * kXcds + (b % kXcds);
 }
 
+constexpr int64_t kMaxChunkLevelBlocks = (int64_t)0xffffffffu / kBlock;
+
+static inline int64_t chunk_level_blocks(int64_t chunks, int levels) {
+  return ceil_div(chunks, (int64_t)kXcds) * kXcds * levels;
+}
+
 static inline int chunk_level_grid(int64_t chunks, int levels, dim3* grid) {
-  const int64_t blocks = ceil_div(chunks, (int64_t)kXcds) * kXcds * levels;
-  NA_CHECK_ARG(blocks * kBlock <= (int64_t)0xffffffffu, "n too large for one launch");
+  const int64_t blocks = chunk_level_blocks(chunks, levels);
+  NA_CHECK_ARG(blocks <= kMaxChunkLevelBlocks, "n too large for one launch");
   *grid = dim3((unsigned)blocks);
   return NA_OK;
 }
@@ -417,18 +423,19 @@ sdf_taps_input_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n, fl
 // lattice points; the five contributions to each corner are summed in
 // registers.  Two threads own one feature of one level for `run` consecutive
 // points (consecutive samples of a ray; the launch tunable taps_bwd.run,
-// default 4): while their boxes share one anchor
+// default 4, 16 from the tune cache): while their boxes share one anchor
 // the sums keep accumulating, and each touched corner gets one atomic when the
 // anchor changes or the run ends.  At coarse levels, where neighbouring
 // samples share cells and atomics to one address would otherwise queue, this
 // removes most of the atomics.  What remains is bounded by the atomics' read-modify-write
 // of scattered entries (fine levels touch up to 27 corners of a box), so two lanes per
-// feature share a box and send neighbours in x together; the vector work that both
-// repeat is below a quarter of the time.  786,432 points, 8 features, bf16 rows: 3.33 ms
-// with one lane per feature and corner by corner, 2.90 ms; 49,152 points, 4 features,
-// float32: 261 us and 198 us.  The price is paid where samples lie so close that few
-// atomics remain: a dense step at the initial field takes 1.85 ms, 1.66 with one lane;
-// choosing per wave by whether its runs leave their cell did not win it back (1.84).  When a level's cells spread wider than one cell
+// feature share a box and send neighbours in x together; they also share the loads of a
+// point's rows, which is what bounds the launch where boxes last.  786,432 points of a
+// packed batch, 8 features, bf16 rows: 3.36 ms with one lane per feature and corner by corner,
+// 2.69 with two lanes that each load all rows, 2.50; samples of a dense step at the initial field,
+// which lie close: 2.14, 2.32 and 1.81; 49,152 points, 4 features, float32: 266, 200 and 197 us.
+// Forming a point's coordinates and weights once for all its lanes, in LDS, was no faster (1.87
+// ms dense).  When a level's cells spread wider than one cell
 // (an epsilon larger than the finest active cell), that point falls back to
 // one atomic per point and corner.
 
@@ -474,6 +481,18 @@ __device__ __attribute__((always_inline)) inline void taps_flush(float* gtab, co
   }
 }
 
+// The value of lane ^ F (F = 1, 2, 4 or 8) through DPP.
+template <int F>
+__device__ inline float lane_xor(float v) {
+  int u = __float_as_int(v);
+  if constexpr (F == 1) u = __builtin_amdgcn_mov_dpp(u, 0xB1, 0xf, 0xf, false);       // quad 1, 0, 3, 2
+  else if constexpr (F == 2) u = __builtin_amdgcn_mov_dpp(u, 0x4E, 0xf, 0xf, false);  // quad 2, 3, 0, 1
+  else if constexpr (F == 4)  // 7 - i in eight lanes, then 3 - i in the quad
+    u = __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(u, 0x141, 0xf, 0xf, false), 0x1B, 0xf, 0xf, false);
+  else u = __builtin_amdgcn_mov_dpp(u, 0x128, 0xf, 0xf, false);  // rotated by 8 in sixteen lanes
+  return __int_as_float(u);
+}
+
 // P2: the volume range is a positive normal power of two, 2^(-vshift) of the
 // unit cube, and coordinates normalise by an exact exponent shift (no division
 // code in that instantiation).
@@ -482,14 +501,14 @@ __global__ void __launch_bounds__(kBlock)
 hashgrid_taps_bwd_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n, float vmin,
                          float vrange, int vshift, float eps, const TD* __restrict__ dyc,
                          const TD* __restrict__ dyt, const TD* __restrict__ dyq, int64_t ld,
-                         float* __restrict__ grad, int inc, int run, int active, int64_t chunk0) {
+                         float* __restrict__ grad, int inc, int run, int active) {
   auto unit = [&](float v) -> float {
     return P2 ? ldexpf(v - vmin, vshift) : normalize_coord(v, vmin, vrange);
   };
   int64_t chunk;
   int l;
   chunk_level(active, chunk, l);
-  const int64_t tid = (chunk0 + chunk) * kBlock + threadIdx.x;
+  const int64_t tid = chunk * kBlock + threadIdx.x;
   const int64_t i0 = (tid / (2 * F)) * run;
   const int f = (int)(tid % F), par = (int)(tid / F) & 1;
   if (i0 >= n) return;
@@ -500,21 +519,21 @@ hashgrid_taps_bwd_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n,
   uint32_t mask = 0;
   int blo[3] = {0, 0, 0};
   const int64_t iend = i0 + run < n ? i0 + run : n;
-  // the rows and coordinates of point i + 1 are loaded while point i is processed
+  // A point's six rows are shared out between the lanes of a feature: the even one loads
+  // the centre's and the first two taps', the odd one the shared and the last two taps', and
+  // they exchange them (half the load instructions, which bound the launch where boxes last).
+  // The rows of point i + 1 are loaded while point i is processed.
   struct Rows {
-    float c, t[4], q, x[3];
+    float one, tap[2], x[3];
   };
+  const bool shared_row = inc && dyq;
+  const TD* one0 = (par && shared_row ? dyq : dyc) + col;
+  const TD* tap0 = dyt + (inc ? 2 * par * ld : 2 * par * n * ld) + col;
+  const int64_t tap_point = inc ? 4 * ld : ld, tap_row = inc ? ld : n * ld;
   auto fetch = [&](int64_t i, Rows& r) {
-    if (inc) {
-      r.q = dyq ? scalar_io<TD>::load(dyq + i * ld + col) : 0.0f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) r.t[t] = scalar_io<TD>::load(dyt + (4 * i + t) * ld + col);
-    } else {
-      r.q = 0.0f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) r.t[t] = scalar_io<TD>::load(dyt + ((int64_t)t * n + i) * ld + col);
-    }
-    r.c = scalar_io<TD>::load(dyc + i * ld + col);
+    r.one = scalar_io<TD>::load(one0 + i * ld);
+    r.tap[0] = scalar_io<TD>::load(tap0 + i * tap_point);
+    r.tap[1] = scalar_io<TD>::load(tap0 + i * tap_point + tap_row);
 #pragma unroll
     for (int k = 0; k < 3; ++k) r.x[k] = x[i * 3 + k];
   };
@@ -522,20 +541,24 @@ hashgrid_taps_bwd_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n,
   fetch(i0, nxt);
   for (int64_t i = i0; i < iend; ++i) {
     const Rows cur = nxt;
+    const float one = lane_xor<F>(cur.one), tap[2] = {lane_xor<F>(cur.tap[0]), lane_xor<F>(cur.tap[1])};
     if (i + 1 < iend) fetch(i + 1, nxt);
     float g[5];
+    g[0] = par ? one : cur.one;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      g[1 + t] = par ? tap[t] : cur.tap[t];
+      g[3 + t] = par ? cur.tap[t] : tap[t];
+    }
     if (inc) {
       // increments: tap rows point-major, gradients of the inputs D_t = X(x + eps k_t)
       // - X(x) (dyt, plus the point row dyq, the gradient of sum_t D_t, shared by the
       // four taps); the centre row holds the gradient of the centre input alone, so
       // the centre's corners receive g_c - sum_t g_t (formed here in fp32)
+      const float q = shared_row ? (par ? cur.one : one) : 0.0f;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) g[1 + t] = cur.t[t] + cur.q;
-      g[0] = cur.c - ((g[1] + g[2]) + (g[3] + g[4]));
-    } else {
-      g[0] = cur.c;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) g[1 + t] = cur.t[t];
+      for (int t = 0; t < 4; ++t) g[1 + t] += q;
+      g[0] -= (g[1] + g[2]) + (g[3] + g[4]);
     }
     if (g[0] == 0.0f && g[1] == 0.0f && g[2] == 0.0f && g[3] == 0.0f && g[4] == 0.0f) continue;
     // Per axis the five evaluations take three coordinates: the centre's and
@@ -900,23 +923,19 @@ static int launch_taps_bwd(const na_grid_desc* d, const float* x, int64_t n, flo
                            hipStream_t s) {
   // the scatter orders the cells of x - eps, x, x + eps along each axis
   NA_CHECK_ARG(eps >= 0.0f, "tap epsilon must be non-negative");
-  const int run = (int)tune_value(TUNE_TAPS_BWD_RUN);
+  int run = (int)tune_value(TUNE_TAPS_BWD_RUN);
   uint32_t vb;
   memcpy(&vb, &vrange, 4);
   const bool p2 = (vb & 0x807fffffu) == 0u && (vb >> 23) != 0u;  // positive normal power of two
   const int vshift = p2 ? 127 - (int)(vb >> 23) : 0;
   auto kernel = p2 ? hashgrid_taps_bwd_kernel<F, TD, true> : hashgrid_taps_bwd_kernel<F, TD, false>;
-  const int64_t chunks = ceil_div(ceil_div(n, (int64_t)run) * 2 * F, kBlock);
-  // the limit on n is that of one lane per feature; with two, up to two launches cover it
+  // more points than a grid of these runs holds: runs of twice the length, once
+  auto chunks = [&]() { return ceil_div(ceil_div(n, (int64_t)run) * 2 * F, kBlock); };
+  if (chunk_level_blocks(chunks(), active) > kMaxChunkLevelBlocks) run *= 2;
   dim3 grid;
-  if (int st = chunk_level_grid(ceil_div(chunks, (int64_t)2), active, &grid)) return st;
-  const int64_t per_launch = ceil_div(ceil_div(chunks, (int64_t)2), (int64_t)kXcds) * kXcds;
-  const bool one = chunk_level_grid(chunks, active, &grid) == NA_OK;
-  for (int64_t c0 = 0; c0 < chunks; c0 += one ? chunks : per_launch) {
-    if (!one) chunk_level_grid(per_launch, active, &grid);
-    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, *d, x, n, vmin, vrange, vshift, eps,
-                       (const TD*)dyc, (const TD*)dyt, (const TD*)dyq, ld, grad, inc, run, active, c0);
-  }
+  if (int st = chunk_level_grid(chunks(), active, &grid)) return st;
+  hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, *d, x, n, vmin, vrange, vshift, eps,
+                     (const TD*)dyc, (const TD*)dyt, (const TD*)dyq, ld, grad, inc, run, active);
   NA_CHECK_LAUNCH();
   return NA_OK;
 }
