@@ -5,7 +5,7 @@ of samples per thread, the tap-increment backward's launch form and workgroups
 per CU, the persistent packed launches' rays per workgroup and workgroups per CU)
 have a best value that depends on the device and on the shape of the work.  `tune()` times every candidate of each on
 the workload it serves -- the train step's samples (8192 rays x 96 samples,
-ray-ordered, as the renderer hands them over) and the ragged packed batch
+ray-ordered, as the renderer hands them over, and evenly spaced) and the ragged packed batch
 (65,536 rays, 0..192 samples) -- with HIP events on the launching stream, and
 keeps the fastest.  The winners are stored per device architecture in
 `tune_cache.json` beside this file; `_lib.load()` applies the entries for the
@@ -164,14 +164,20 @@ def tune(dev=None, write=True, path=CACHE_PATH):
     vmin, vmax = enc.vol_range
     g = torch.Generator(device=dev).manual_seed(1)
 
+    # and the same rows at samples spaced evenly along the rays, as in a packed batch (the
+    # hierarchical samples of the step lie close together)
+    k = torch.arange(P // 8192, device=dev)[None, :, None] * (2.0 / (P // 8192)) + 2.0
+    even = (c[:, None] + v[:, None] * k).reshape(-1, 3).contiguous()
+
     def scatter():
-        _lib.call("na_sdf_taps_bwd", ctypes.byref(enc.desc), _lib.ptr(pts), P, float(vmin),
-                  float(vmax), float(eps), _lib.ptr(dXc), _lib.ptr(dXt),
-                  _lib.ptr(dXq) if dXq is not None else None, _lib.dtype_code(dXc.dtype), ld,
-                  _lib.ptr(grad), int(enc.active_levels), int(inc), _lib.stream_of(pts))
+        for at in (pts, even):
+            _lib.call("na_sdf_taps_bwd", ctypes.byref(enc.desc), _lib.ptr(at), P, float(vmin),
+                      float(vmax), float(eps), _lib.ptr(dXc), _lib.ptr(dXt),
+                      _lib.ptr(dXq) if dXq is not None else None, _lib.dtype_code(dXc.dtype), ld,
+                      _lib.ptr(grad), int(enc.active_levels), int(inc), _lib.stream_of(pts))
     rec = _sweep("taps_bwd.run", scatter)
-    rec["workload"] = (f"na_sdf_taps_bwd on a BF16 train step's own inputs ({P} samples of "
-                       "8192 rays, the step's dL/dy rows)")
+    rec["workload"] = (f"na_sdf_taps_bwd on a BF16 train step's dL/dy rows ({P} samples of "
+                       "8192 rays): its own samples, and samples spaced evenly along the rays")
     out["taps_bwd.run"] = rec
     del cap, dXc, dXt, dXq, grad
 

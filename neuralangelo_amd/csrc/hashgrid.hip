@@ -423,7 +423,7 @@ sdf_taps_input_kernel(na_grid_desc d, const float* __restrict__ x, int64_t n, fl
 // lattice points; the five contributions to each corner are summed in
 // registers.  Two threads own one feature of one level for `run` consecutive
 // points (consecutive samples of a ray; the launch tunable taps_bwd.run,
-// default 4, 16 from the tune cache): while their boxes share one anchor
+// default 4, 12 from the tune cache): while their boxes share one anchor
 // the sums keep accumulating, and each touched corner gets one atomic when the
 // anchor changes or the run ends.  At coarse levels, where neighbouring
 // samples share cells and atomics to one address would otherwise queue, this
