@@ -55,7 +55,7 @@ __device__ inline float sv_point_weight(const bf16_t* w, int K, int k) {
 
 // T: table and weight type (float: three planes and split weights; bf16: one plane).
 // F features per level, L levels, K = L F (a multiple of 16); NB 32-column blocks per
-// wave (hidden width 128 NB).
+// wave (hidden width 32 NB WAVES).
 template <typename T, int F, int K, int NB, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, 4) sdf_value_kernel(na_grid_desc d, SdfValueParams p) {
   constexpr bool F32 = sizeof(T) == 4;
@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(64 * WAVES, 4) sdf_value_kernel(na_grid_desc d
   __syncthreads();
   if constexpr (F32) {
     // values that are not finite, or too large to split into bf16 parts: the tile again
-    // in float32, a thread per point and quarter of the columns
+    // in float32, a thread per point and wave, which takes its own columns
     if (__builtin_expect(s_odd != 0, 0)) {
       const int pt = tid & 63;
       float total = 0.0f;

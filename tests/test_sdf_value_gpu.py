@@ -88,3 +88,23 @@ def test_sdf_value_unsplittable(value):
         assert (torch.sign(got[big]) == torch.sign(ref[big])).all() and (got[big].abs() > 1e29).all()
     else:
         assert (got - ref).abs().max() <= 1e-3
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("F,hidden", [(8, 256), (8, 128), (4, 256), (4, 128)])
+def test_sdf_value_recomputed_tile(F, hidden, value):
+    """One bad entry of a float32 table: its tile is formed again in float32, the points that
+    read the entry follow it, and the tile's other points keep their accuracy."""
+    enc, w, g = _setup(F, hidden, torch.float32, 16)
+    x = (torch.rand(200, 3, generator=g) * 2 - 1).cuda()
+    with torch.no_grad():
+        idx, wt = enc.corners((x + 1.0) / 2.0)
+        entry = int(idx[70, 15, 3])  # a corner of point 70 at the finest level
+        enc.params.view(-1, F)[entry, F - 1] = value
+        hit = (idx == entry).flatten(1).any(1)
+        assert hit[70] and hit[64:128].sum() < 8
+        got = Fn.sdf_forward_nograd(enc, w, x).double()
+        ref, e = _reference(enc, w, x)
+    assert ((got - ref).abs() <= e)[~hit].all()
+    if abs(value) != 3.4e38:
+        assert not got[hit].isfinite().any() and not ref[hit].isfinite().any()
