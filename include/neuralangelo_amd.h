@@ -193,8 +193,8 @@ typedef struct na_gemm_args {
 int na_gemm(const na_gemm_args* args, na_stream_t stream);
 
 /* The _slots forms of the calls whose workgroups each add to the same few addresses when
- * they end (column sums, narrow weight gradients).  One address takes an atomic about every
- * 0.18 us, so 512 workgroups that end together wait 90 us for each other.  Here
+ * they end (column sums, narrow weight gradients).  A cache line takes an atomic request about
+ * every 22 ns, so workgroups that end together wait for each other.  Here
  * they add to copy (workgroup mod slots) of each such destination, `slot_stride` floats after
  * the previous one; the caller zeroes slots copies and sums them afterwards.  slots = 1 is
  * the plain call. */

@@ -68,10 +68,10 @@ struct GemmParams {
   EpiParams e;
 };
 
-// Sums that every workgroup adds to the same few addresses when it ends: one address takes
-// an atomic about every 0.18 us, so 512 workgroups that end together wait 90 us for
-// each other.  The caller can pass several zeroed copies of the destination,
-// `stride` floats apart, and sum them afterwards; workgroups take them in turn.
+// Sums that every workgroup adds to the same few addresses when it ends: a cache line takes
+// an atomic request about every 22 ns, so 512 workgroups that end together with 8
+// requests a line wait 90 us for each other.  The caller can pass several zeroed copies of the
+// destination, `stride` floats apart, and sum them afterwards; workgroups take them in turn.
 __device__ inline int64_t slot_offset(int slots, int64_t stride) {
   return slots > 1 ? (int64_t)(blockIdx.x % (uint32_t)slots) * stride : 0;
 }
@@ -1750,8 +1750,9 @@ gemm_bf16_nn_persist_kernel(GemmParams p) {
 // ---------------------------------------------------------------------------
 // float32 GEMM on the bf16 matrix cores.
 //
-// A float32 value is the exact sum of three bf16 values, x = x1 + x2 + x3 (x1 =
-// bf16(x), x2 = bf16(x - x1), x3 = the rest: 3 x 8 significand bits), so a
+// A float32 value from 2^-109 up is the exact sum of three bf16 values, x = x1 + x2 + x3 (x1 =
+// bf16(x), x2 = bf16(x - x1), x3 = the rest: 3 x 8 significand bits; a smaller value's
+// last bits lie below bf16's range and are lost), so a
 // product is x y = x1 y1 + (x1 y2 + x2 y1) + (x2 y2 + x1 y3 + x3 y1) up to terms of
 // 2^-25 |x y| and below, under the rounding of one float32 multiply.  A 16-wide
 // step of the bf16 instruction six times takes 192 cycles where the float32
@@ -1775,8 +1776,8 @@ gemm_bf16_nn_persist_kernel(GemmParams p) {
 // Rows x columns x K, float32 instruction -> here: 2,146,689 x 256 x 136 2.18 -> 1.43 ms,
 // 98,304 x 256 x 280 168 -> 95 us, 49,152 x 256 x 256 84 -> 53 us, 4,096 x 256 x 68 28 -> 8 us;
 // transposed (weight gradients; before, also too few parts of the sum): 256 x 136 over
-// 196,608 rows 427 -> 162 us, 256 x 280 over 28,800 rows 302 -> 58 us, 256 x 84 over 3,200
-// rows 380 -> 14 us.
+// 196,608 rows 427 -> 149 us, 256 x 280 over 20,000 rows 319 -> 38 us, 256 x 84 over 3,200
+// rows 380 -> 15 us.
 constexpr int kF3BK = 32, kF3BM = 128;
 
 // One operand tile of R rows x 32 k, float32 chunks in registers.  Rows past the
@@ -1878,7 +1879,8 @@ __device__ inline float f3_at(const float* __restrict__ X, int64_t ld, int64_t r
 // Where the outputs go.  F3_ROWS: a lane holds 16 columns of one row per 32 x 32 block
 // (the weights are the first MFMA operand) and finishes them in registers, 8 at a
 // time, with 16-byte loads and stores.  F3_ATOMIC: a lane holds one column (rows in
-// registers), so an atomic instruction covers whole row segments.  F3_GENERAL: the
+// registers), so an atomic instruction, or the store of a partial sum, covers whole row
+// segments.  F3_GENERAL: the
 // staged epilogue, for unaligned rows, widths that are not multiples of 8 and the
 // rare epilogue terms.  Each mode takes each operand layout it is launched with below.
 enum F3Mode : int { F3_ROWS, F3_ATOMIC, F3_GENERAL };

@@ -9,7 +9,8 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((ext_vector_type(8))) float f32x8_t;
 
-// x = h[0] + h[1] + h[2] exactly, three bf16 values (rounded to nearest)
+// x = h[0] + h[1] + h[2], three bf16 values (rounded to nearest); exact from 2^-109 up, below
+// which the last part leaves bf16's range
 __device__ inline void split3(const f32x8_t& x, bf16x8_t (&h)[3]) {
   h[0] = __builtin_convertvector(x, bf16x8_t);
   const f32x8_t r = x - __builtin_convertvector(h[0], f32x8_t);
