@@ -3567,12 +3567,18 @@ extern "C" int na_linear_narrow_bwd_slots(const void* X, int64_t ldx, int32_t x_
   int64_t waves = ceil_div(M, 16);
   if (waves > 4096) waves = 4096;
   dim3 grid8((unsigned)ceil_div(waves, 8));
+  // One output over many float32 rows of up to 256 columns, in and out: LDS that keeps a second
+  // workgroup off the CU, since two resident ones mix more streams of reads and writes
+  // (800,000 x 256: 377 us with two, 356 with one; 400,000 187 and 179; 100,000 50 and 53;
+  // more outputs, bf16 and 128 columns gain nothing or lose).
+  const size_t alone = N == 1 && dX && x_dtype == NA_F32 && K > 128 && K <= 256 &&
+                       M >= (int64_t)1 << 18 ? 66 * 1024 : 0;
   hipStream_t s = (hipStream_t)stream;
   // X is the only row operand: no dX accumulation, and the derivative (if
   // any) is read from X itself
   const bool x_only = !add_dx && (!dX || !dact || (Y == X && ldy == ldx && y_dtype == x_dtype));
 #define NA_NBWD_L(TX, TDX, KC, NM, XO)                                                         \
-  hipLaunchKernelGGL((narrow_bwd_vec_kernel<TX, TDX, KC, NM, XO>), grid8, dim3(512), 0, s,     \
+  hipLaunchKernelGGL((narrow_bwd_vec_kernel<TX, TDX, KC, NM, XO>), grid8, dim3(512), alone, s, \
                      (const TX*)X, ldx, M, K, W, N, dpre, dW, db, (TDX*)dX, lddx, add_dx, Y,   \
                      ldy, y_dtype, dact, act_beta, dx_colsum, slots, slot_stride)
 #define NA_NBWD(TX, TDX, KC)                                                                   \
