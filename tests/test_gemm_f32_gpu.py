@@ -146,3 +146,17 @@ def test_split_k_of_one_is_one_addition():
         out.append(dW)
     assert all(torch.equal(o, out[0]) for o in out[1:])
     assert ((out[0].double() - D.double() @ X.double().t()).abs() <= bound(D, X, rows)).all()
+
+
+@pytest.mark.parametrize("rows, N, K, parts", [(3204, 64, 84, 3), (500, 130, 257, 40), (36, 8, 20, 7)])
+def test_split_k_parts_without_a_workspace(rows, N, K, parts):
+    """The caller's parts add atomically, also where some of them hold no rows."""
+    g = torch.Generator().manual_seed(parts)
+    D, dpre, ldd = operand(N, rows, 1, g)
+    X, x, ldx = operand(K, rows, 1, g)
+    dW = torch.full((N, K), 0.5, device="cuda")
+    Fn.gemm(dpre, ldd, 1, x, ldx, 1, N, K, rows, dW, K, epilogue=NA_EPI_ATOMIC, split_k=parts,
+            wgrad_partials=False)
+    ref, size = D.double() @ X.double().t(), D.double().abs() @ X.double().abs().t()
+    slack = (parts + 2) * 2.0 ** -24 * (0.5 + size)
+    assert ((dW.double() - 0.5 - ref).abs() <= bound(D, X, rows) + slack).all()
